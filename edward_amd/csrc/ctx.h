@@ -61,6 +61,15 @@ struct DevBuf {
   }
 };
 
+// Plan of the one-pass few-chain gradient (few_chains.h) for the bound data
+// and the current chain count; off where it does not apply.
+struct FewPlan {
+  bool on = false;
+  int DP = 0;              // columns of the X it reads
+  int splits = 0;          // row ranges
+  int64_t rows_per_split = 0;
+};
+
 }  // namespace edhmc
 
 struct edhmc_ctx {
@@ -89,7 +98,10 @@ struct edhmc_ctx {
   edhmc::DevBuf ratio;   // [C] FP64 Metropolis log ratio of the last HMC transition
   // ---- gradient scratch ----
   edhmc::DevBuf Rt, Gpart, llpart, ll;
-  int ksplit = 1;
+  int ksplit = 1;        // partial gradients in Gpart, g_ld chains x D_pad apart
+  int64_t g_ld = 0;
+  edhmc::FewPlan few;
+  edhmc::DevBuf Xs;      // X with few.DP < D_pad columns (few-chain gradient)
   int n_tiles1 = 0;      // GEMM1 column tiles (= llpart leading dim)
   // ---- moments ----
   bool mom_on = false;

@@ -20,6 +20,7 @@
 #include "ctx.h"
 #include "gemm_nt.h"
 #include "gemm2_dma.h"
+#include "few_chains.h"
 #include "philox.h"
 #include "transform.h"
 
@@ -492,7 +493,8 @@ struct ChainArgs {
   float half, full;         // fl32(eps/2), fl32(eps)
   const float* r_fed; const double* u_fed;
   uint64_t seed, counter;
-  const float* Gpart; int ksplit;
+  const float* Gpart; int ksplit;   // partial gradients, g_stride floats apart
+  int64_t g_stride;
   const double* ll;         // [C_pad] reduced log-likelihood
   float lik_weight;         // multiplies the likelihood (scale of the SG samplers; 1 for HMC)
   const float* beta;        // per-chain inverse temperature of the MH ratio (null = 1)
@@ -588,22 +590,66 @@ __global__ void __launch_bounds__(kChainThreads) chain_begin_kernel(ChainArgs a)
 }
 
 __device__ inline float gsum(const ChainArgs& a, int c, int d) {
-  const int64_t stride = (int64_t)a.C_pad * a.D_pad;
   const float* p = a.Gpart + (int64_t)c * a.D_pad + d;
   float s = 0.0f;
-  for (int q = 0; q < a.ksplit; ++q) s += p[q * stride];
+  for (int q = 0; q < a.ksplit; ++q) s += p[q * a.g_stride];
   return a.lik_weight * s;
 }
 
+// The likelihood gradient of chain c for every coordinate, by the whole
+// workgroup of NT threads: 16-byte loads, the partials dealt round-robin to
+// NT / (D_pad / 4) groups of threads and the groups' sums combined in a fixed
+// order.  For the few-chain gradient, which leaves up to a thousand partials
+// per chain.  D_pad <= 256.
+struct CoopG {
+  const float* lds;
+  float w;
+  __device__ float operator()(int d) const { return w * lds[d]; }
+};
+template <int NT>
+__device__ inline CoopG gsum_block(const ChainArgs& a, int c) {
+  __shared__ __align__(16) float part[4 * NT];
+  __shared__ float tot[256];
+  const int d4 = a.D_pad >> 2, ng = NT / d4;
+  const int t = threadIdx.x, gq = t / d4, l = t - gq * d4;
+  if (gq < ng) {
+    const f32x4_t* p = (const f32x4_t*)(a.Gpart + (int64_t)c * a.D_pad) + l;
+    const int64_t st = a.g_stride >> 2;
+    f32x4_t s = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 8
+    for (int q = gq; q < a.ksplit; q += ng) s += p[q * st];
+    *(f32x4_t*)(part + 4 * t) = s;
+  }
+  __syncthreads();
+  for (int d = t; d < a.D_pad; d += NT) {
+    float s = 0.0f;
+    for (int q = 0; q < ng; ++q) s += part[q * a.D_pad + d];
+    tot[d] = s;
+  }
+  __syncthreads();
+  return CoopG{tot, a.lik_weight};
+}
+struct ThreadG {
+  const ChainArgs& a;
+  int c;
+  __device__ float operator()(int d) const { return gsum(a, c, d); }
+};
+template <int NT, bool COOP>
+__device__ inline auto chain_gradient(const ChainArgs& a, int c) {
+  if constexpr (COOP) return gsum_block<NT>(a, c);
+  else return ThreadG{a, c};
+}
 
 // Middle of the trajectory: gradient at the new z, r += eps/2 g twice
 // (end of this step, start of the next), drift.
-__global__ void __launch_bounds__(kChainThreads) chain_mid_kernel(ChainArgs a) {
+template <int NT, bool COOP>
+__global__ void __launch_bounds__(NT) chain_mid_kernel(ChainArgs a) {
   const int c = blockIdx.x;
-  for (int d = threadIdx.x; d < a.D; d += kChainThreads) {
+  const auto gl = chain_gradient<NT, COOP>(a, c);
+  for (int d = threadIdx.x; d < a.D; d += NT) {
     const int64_t idx = (int64_t)c * a.D_pad + d;
     const float zv = a.z[idx];
-    const float gv = grad_u(a, d, zv, gsum(a, c, d));
+    const float gv = grad_u(a, d, zv, gl(d));
     a.g[idx] = gv;
     if (a.rec_W) {
       a.rec_W[(int64_t)c * a.D + d] = zv;
@@ -621,14 +667,14 @@ __global__ void __launch_bounds__(kChainThreads) chain_mid_kernel(ChainArgs a) {
 
 // Shared end of trajectory: last half kick, ratio, accept, select, store.
 // `g_at` supplies the gradient at the end point (exact or surrogate).
-template <typename GradAt>
+template <int NT, typename GradAt>
 __device__ inline void chain_accept(const ChainArgs& a, GradAt g_at) {
-  __shared__ double red[kChainThreads / 64];
+  __shared__ double red[NT / 64];
   __shared__ int acc_flag;
   const int c = blockIdx.x;
   double kl = 0.0, plp = 0.0;
   int bad = 0;
-  for (int d = threadIdx.x; d < a.D; d += kChainThreads) {
+  for (int d = threadIdx.x; d < a.D; d += NT) {
     const int64_t idx = (int64_t)c * a.D_pad + d;
     const float zv = a.z[idx];
     const float gv = g_at(c, d, idx, zv);
@@ -639,10 +685,10 @@ __device__ inline void chain_accept(const ChainArgs& a, GradAt g_at) {
     plp += prior_logp(a, d, zv);
     if (!isfinite(zv) || !isfinite(gv)) bad = 1;
   }
-  kl = block_sum_f64<kChainThreads>(kl, red);
-  plp = block_sum_f64<kChainThreads>(plp, red);
+  kl = block_sum_f64<NT>(kl, red);
+  plp = block_sum_f64<NT>(plp, red);
   const double ll = (double)a.lik_weight * a.ll[c];
-  const double nbad = block_sum_f64<kChainThreads>((double)bad, red);
+  const double nbad = block_sum_f64<NT>((double)bad, red);
   if (threadIdx.x == 0) {
     const double logpL = ll + plp;
     const double ratio = a.K0[c] - 0.5 * kl + logpL - a.logp[c];
@@ -658,7 +704,7 @@ __device__ inline void chain_accept(const ChainArgs& a, GradAt g_at) {
   }
   __syncthreads();
   const int acc = acc_flag;
-  for (int d = threadIdx.x; d < a.D; d += kChainThreads) {
+  for (int d = threadIdx.x; d < a.D; d += NT) {
     const int64_t idx = (int64_t)c * a.D_pad + d;
     float zv;
     if (acc) {
@@ -679,27 +725,29 @@ __device__ inline void chain_accept(const ChainArgs& a, GradAt g_at) {
   }
 }
 
-__global__ void __launch_bounds__(kChainThreads) chain_last_kernel(ChainArgs a) {
-  chain_accept(a, [&](int c, int d, int64_t, float zv) {
-    return grad_u(a, d, zv, gsum(a, c, d));
-  });
+template <int NT, bool COOP>
+__global__ void __launch_bounds__(NT) chain_last_kernel(ChainArgs a) {
+  const auto gl = chain_gradient<NT, COOP>(a, blockIdx.x);
+  chain_accept<NT>(a, [&](int, int d, int64_t, float zv) { return grad_u(a, d, zv, gl(d)); });
 }
 
 // Evaluation at the current z: gradient + log joint into the state (and
 // optional outputs).
-__global__ void __launch_bounds__(kChainThreads) chain_eval_kernel(ChainArgs a) {
-  __shared__ double red[kChainThreads / 64];
+template <int NT, bool COOP>
+__global__ void __launch_bounds__(NT) chain_eval_kernel(ChainArgs a) {
+  __shared__ double red[NT / 64];
   const int c = blockIdx.x;
+  const auto gl = chain_gradient<NT, COOP>(a, c);
   double plp = 0.0;
-  for (int d = threadIdx.x; d < a.D; d += kChainThreads) {
+  for (int d = threadIdx.x; d < a.D; d += NT) {
     const int64_t idx = (int64_t)c * a.D_pad + d;
     const float zv = a.z[idx];
-    const float gv = grad_u(a, d, zv, gsum(a, c, d));
+    const float gv = grad_u(a, d, zv, gl(d));
     a.g[idx] = gv;
     if (a.grad_out) a.grad_out[(int64_t)c * a.D + d] = gv;
     plp += prior_logp(a, d, zv);
   }
-  plp = block_sum_f64<kChainThreads>(plp, red);
+  plp = block_sum_f64<NT>(plp, red);
   const double ll = (double)a.lik_weight * a.ll[c];
   if (threadIdx.x == 0) {
     a.logp[c] = ll + plp;
@@ -1018,11 +1066,34 @@ static ChainArgs chain_args(edhmc_ctx* ctx) {
     a.plnorm = (const double*)ctx->plnorm.p;
   }
   a.Gpart = (const float*)ctx->Gpart.p; a.ksplit = ctx->ksplit;
+  a.g_stride = ctx->g_ld * ctx->D_pad;
   a.ll = (const double*)ctx->ll.p;
   a.lik_weight = ctx->lik_weight;
   a.ndiv = (int32_t*)ctx->ndiv.p;
   a.ratio_out = (double*)ctx->ratio.p;
   return a;
+}
+
+// Launch one of the chain kernels that sum the partial gradients: by the
+// whole workgroup after a few-chain gradient, a thread per coordinate
+// otherwise.
+enum ChainKernel { kChainMid, kChainLast, kChainEval };
+static int launch_chain(edhmc_ctx* ctx, ChainKernel k, const ChainArgs& a, hipStream_t st) {
+  auto go = [&](auto nt, auto coop) {
+    constexpr int NT = decltype(nt)::value;
+    constexpr bool COOP = decltype(coop)::value;
+    const dim3 grid(ctx->C), block(NT);
+    if (k == kChainMid) hipLaunchKernelGGL((chain_mid_kernel<NT, COOP>), grid, block, 0, st, a);
+    else if (k == kChainLast) hipLaunchKernelGGL((chain_last_kernel<NT, COOP>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((chain_eval_kernel<NT, COOP>), grid, block, 0, st, a);
+  };
+  using std::integral_constant;
+  using std::false_type;
+  using std::true_type;
+  if (!ctx->few.on) go(integral_constant<int, kChainThreads>{}, false_type{});
+  else go(integral_constant<int, 1024>{}, true_type{});
+  static const char* const names[] = {"chain_mid", "chain_last", "chain_eval"};
+  return check_launch(ctx, names[k]);
 }
 
 // ll[c] = sum over the n_tiles row tiles of llpart[t][c] (fixed order).
@@ -1156,7 +1227,32 @@ static bool ws_grad_ok(const edhmc_ctx* ctx) {
   return ws_forward_ok(ctx);
 }
 
+// One-pass gradient of a few chains (or, with grad = false, their
+// log-likelihood alone).
+static int few_eval(edhmc_ctx* ctx, bool grad, bool ll, hipStream_t st) {
+  FewArgs a = {};
+  a.X = (const float*)(ctx->few.DP < ctx->D_pad ? ctx->Xs.p : ctx->Xr.p);
+  a.y = (const float*)ctx->y.p;
+  a.W = (const float*)ctx->z_lp.p;
+  a.ldw = ctx->D_pad;
+  a.N = ctx->N;
+  a.rows_per_split = ctx->few.rows_per_split;
+  a.C = ctx->C;
+  a.splits = ctx->few.splits;
+  a.lp = lik_params(ctx);
+  a.Gpart = (float*)ctx->Gpart.p;
+  a.ldg = ctx->D_pad;
+  a.llpart = (double*)ctx->llpart.p;
+  a.ll_ld = ctx->C_pad;
+  {
+    ProfScope ps(ctx, grad ? PK_GEMM_GRAD : PK_GEMM_LL, st);
+    EDHMC_TRY(few_launch(ctx, a, ctx->few.DP, grad, ll, st));
+  }
+  return ll ? ll_reduce(ctx, a.splits, st) : EDHMC_OK;
+}
+
 static int grad_eval(edhmc_ctx* ctx, bool split, bool ll, hipStream_t st) {
+  if (ctx->few.on) return few_eval(ctx, true, ll, st);
   if (ctx->cdt == EDHMC_BF16) {
     if (split) {
       if (ws_grad_ok(ctx)) {
@@ -1202,7 +1298,7 @@ int glm_grad_eval_offset(edhmc_ctx* ctx, const float* goff, int64_t goff_ld, con
 }
 
 // Buffers the chain-level engines above the GLM need to size their state.
-int glm_ensure_chains(edhmc_ctx* ctx, int C);
+int glm_ensure_chains(edhmc_ctx* ctx, int C, hipStream_t st);
 
 // ---------------------------------------------------------------------------
 // W-stationary forward log-likelihood (Bernoulli, bf16 X, hi/lo W planes):
@@ -1836,6 +1932,7 @@ static int launch_ws_forward(edhmc_ctx* ctx, hipStream_t st, bool wr, int planes
 
 // Forward only (log-likelihood partials, no residuals) at z_lp, exact form.
 int glm_forward_ll(edhmc_ctx* ctx, hipStream_t st) {
+  if (ctx->few.on) return few_eval(ctx, false, true, st);
   if (ws_forward_ok(ctx)) EDHMC_TRY(launch_ws_forward(ctx, st, false));
   else if (ctx->cdt == EDHMC_BF16) EDHMC_TRY((launch_gemm1<bf16_t, CfgP2, 2, false, true>(ctx, st)));
   else EDHMC_TRY((launch_gemm1<float, Cfg1, 1, false, true>(ctx, st)));
@@ -1859,7 +1956,6 @@ int glm_write_lp(edhmc_ctx* ctx, hipStream_t st) {
   return check_launch(ctx, "chain_lp");
 }
 
-static int ensure_chains(edhmc_ctx* ctx, int C);
 
 // Posterior-predictive pass over the bound rows for the S draws in z_lp.
 template <typename T, typename Cfg, int PLANES>
@@ -1908,7 +2004,7 @@ static int launch_predict(edhmc_ctx* ctx, int S, bool want_mean, float* rep, uin
   return EDHMC_OK;
 }
 
-static int ensure_chains(edhmc_ctx* ctx, int C) {
+static int ensure_chains(edhmc_ctx* ctx, int C, hipStream_t st) {
   if (C <= 0) return set_err(ctx, EDHMC_EINVAL, "number of chains must be positive, got %d", C);
   if (ctx->C == C && ctx->z.p) return EDHMC_OK;
   const int C_pad = (int)round_up(C, kChainPad);
@@ -1931,31 +2027,46 @@ static int ensure_chains(edhmc_ctx* ctx, int C) {
   EDHMC_TRY(dev_alloc(ctx, ctx->K0, (size_t)C * 8));
   EDHMC_TRY(dev_alloc(ctx, ctx->ndiv, (size_t)C * 4));
   EDHMC_TRY(dev_alloc(ctx, ctx->ratio, (size_t)C * 8));
-  // rows up to a whole W-stationary tile: its residual epilogue stores the
-  // last tile's rows past N_pad (zeros) without a bounds test
-  EDHMC_TRY(dev_alloc(ctx, ctx->Rt, (size_t)C_pad * round_up(ctx->N_pad, kWsTile) * eb, false));
-  // split-K for GEMM2: aim for >= 2048 workgroups, >= 8 stages per split.
-  const int bn2 = (ctx->D_pad % Cfg1::BN == 0) ? Cfg1::BN : Cfg2S::BN;
-  const int tiles2 = (C_pad / 128) * (ctx->D_pad / bn2);
-  const int kst = (int)(ctx->N_pad * eb / kStageBytes);
-  int ks = (2048 + tiles2 - 1) / tiles2;
-  ks = std::max(1, std::min(ks, std::min(64, kst / 8)));
-  if (ks >= 8) ks = ks / 8 * 8;
-  ctx->ksplit = ks;
-  EDHMC_TRY(dev_alloc(ctx, ctx->Gpart, (size_t)ks * C_pad * ctx->D_pad * 4, false));
   ctx->n_tiles1 = (int)(ctx->N_pad / std::min(Cfg1::BN, CfgP2::BN));   // llpart rows
+  ctx->few = few_plan(ctx, C);
+  if (ctx->few.on) {
+    // no residuals: the row ranges' partial gradients of the C chains
+    ctx->Rt.release();
+    ctx->ksplit = ctx->few.splits;
+    ctx->g_ld = C;
+    ctx->n_tiles1 = std::max(ctx->n_tiles1, ctx->few.splits);
+    if (ctx->few.DP < ctx->D_pad && !ctx->Xs.p) {
+      EDHMC_TRY(dev_alloc(ctx, ctx->Xs, (size_t)ctx->N_pad * ctx->few.DP * 4, false));
+      EDHMC_TRY(few_layout(ctx, (const float*)ctx->Xr.p, ctx->D_pad, ctx->few.DP,
+                           (float*)ctx->Xs.p, st));
+    }
+  } else {
+    // rows up to a whole W-stationary tile: its residual epilogue stores the
+    // last tile's rows past N_pad (zeros) without a bounds test
+    EDHMC_TRY(dev_alloc(ctx, ctx->Rt, (size_t)C_pad * round_up(ctx->N_pad, kWsTile) * eb, false));
+    // split-K for GEMM2: aim for >= 2048 workgroups, >= 8 stages per split.
+    const int bn2 = (ctx->D_pad % Cfg1::BN == 0) ? Cfg1::BN : Cfg2S::BN;
+    const int tiles2 = (C_pad / 128) * (ctx->D_pad / bn2);
+    const int kst = (int)(ctx->N_pad * eb / kStageBytes);
+    int ks = (2048 + tiles2 - 1) / tiles2;
+    ks = std::max(1, std::min(ks, std::min(64, kst / 8)));
+    if (ks >= 8) ks = ks / 8 * 8;
+    ctx->ksplit = ks;
+    ctx->g_ld = C_pad;
+  }
+  EDHMC_TRY(dev_alloc(ctx, ctx->Gpart, (size_t)ctx->ksplit * ctx->g_ld * ctx->D_pad * 4, false));
   EDHMC_TRY(dev_alloc(ctx, ctx->llpart, (size_t)C_pad * ctx->n_tiles1 * 8, false));
   EDHMC_TRY(dev_alloc(ctx, ctx->ll, (size_t)C_pad * 8));
   EDHMC_TRY(dev_alloc(ctx, ctx->ll_split, (size_t)kLLSplit * C_pad * 8, false));
   return EDHMC_OK;
 }
 
-int glm_ensure_chains(edhmc_ctx* ctx, int C) { return ensure_chains(ctx, C); }
+int glm_ensure_chains(edhmc_ctx* ctx, int C, hipStream_t st) { return ensure_chains(ctx, C, st); }
 
 static int do_set_state(edhmc_ctx* ctx, const float* W, int C, hipStream_t st) {
   if (!ctx->bound) return set_err(ctx, EDHMC_ESTATE, "no model bound");
   if (!W) return set_err(ctx, EDHMC_EINVAL, "W is NULL");
-  EDHMC_TRY(ensure_chains(ctx, C));
+  EDHMC_TRY(ensure_chains(ctx, C, st));
   EDHMC_TRY(dev_alloc(ctx, ctx->tmp_count, 4));
   ChainArgs a = chain_args(ctx);
   a.W_in = W;
@@ -1972,8 +2083,7 @@ static int do_set_state(edhmc_ctx* ctx, const float* W, int C, hipStream_t st) {
   }
   EDHMC_TRY(grad_eval(ctx, true, true, st));
   a = chain_args(ctx);
-  hipLaunchKernelGGL(chain_eval_kernel, dim3(C), dim3(kChainThreads), 0, st, a);
-  EDHMC_TRY(check_launch(ctx, "chain_eval"));
+  EDHMC_TRY(launch_chain(ctx, kChainEval, a, st));
   ctx->state_valid = true;
   ctx->g_valid = true;
   surrogate_invalidate(ctx->sur);
@@ -1992,8 +2102,7 @@ static int do_transition(edhmc_ctx* ctx, float eps, int L, const float* r0, cons
     EDHMC_TRY(glm_write_lp(ctx, st));
     EDHMC_TRY(grad_eval(ctx, true, true, st));
     ChainArgs e = chain_args(ctx);
-    hipLaunchKernelGGL(chain_eval_kernel, dim3(ctx->C), dim3(kChainThreads), 0, st, e);
-    EDHMC_TRY(check_launch(ctx, "chain_eval"));
+    EDHMC_TRY(launch_chain(ctx, kChainEval, e, st));
     ctx->g_valid = true;
   }
   surrogate_invalidate(ctx->sur);
@@ -2021,11 +2130,8 @@ static int do_transition(edhmc_ctx* ctx, float eps, int L, const float* r0, cons
         a.rec_G = ctx->rec_G + ctx->rec_count * ctx->D;
         ctx->rec_count += ctx->C;
       }
-      {
-        ProfScope ps(ctx, PK_CHAIN, st);
-        hipLaunchKernelGGL(chain_mid_kernel, dim3(ctx->C), dim3(kChainThreads), 0, st, a);
-      }
-      EDHMC_TRY(check_launch(ctx, "chain_mid"));
+      ProfScope ps(ctx, PK_CHAIN, st);
+      EDHMC_TRY(launch_chain(ctx, kChainMid, a, st));
     }
   }
   a.sample_out = sample_out;
@@ -2037,11 +2143,8 @@ static int do_transition(edhmc_ctx* ctx, float eps, int L, const float* r0, cons
     a.mom_m2 = (double*)ctx->mom_m2.p;
     a.mom_n = ctx->mom_count;
   }
-  {
-    ProfScope ps(ctx, PK_CHAIN, st);
-    hipLaunchKernelGGL(chain_last_kernel, dim3(ctx->C), dim3(kChainThreads), 0, st, a);
-  }
-  return check_launch(ctx, "chain_last");
+  ProfScope ps(ctx, PK_CHAIN, st);
+  return launch_chain(ctx, kChainLast, a, st);
 }
 
 }  // namespace edhmc
@@ -2092,7 +2195,7 @@ edhmc_ctx::~edhmc_ctx() {
   for (hipEvent_t e : prof.pool) (void)hipEventDestroy(e);
   if (sur) surrogate_destroy(sur);
   if (hier) hier_destroy(hier);
-  DevBuf* bufs[] = {&Xr, &Xc, &Xf, &y, &ploc, &pscale, &z, &r, &g, &z0, &g0, &z_lp, &logp, &K0,
+  DevBuf* bufs[] = {&Xr, &Xc, &Xf, &Xs, &y, &ploc, &pscale, &z, &r, &g, &z0, &g0, &z_lp, &logp, &K0,
                     &flag, &ndiv, &ratio, &Rt, &Gpart, &llpart, &ll, &mom_mean, &mom_m2, &tmp_count,
                     &stats_part, &pred_col, &ll_split, &pkind, &plnorm,
                     &newton};
@@ -2150,6 +2253,7 @@ int edhmc_bind_glm(edhmc_ctx* ctx, const void* X, int32_t x_in_dtype, const floa
   ctx->state_valid = false;
   ctx->C = 0;
   ctx->z.release();
+  ctx->Xs.release();   // a copy of the X bound before
   ctx->cdt = compute_dtype;
   ctx->lik = likelihood;
   ctx->lik_scale = lik_scale;
@@ -2268,7 +2372,7 @@ int edhmc_logp(edhmc_ctx* ctx, const float* W, int32_t C, double* logp_out, void
   hipStream_t st = (hipStream_t)stream;
   if (!ctx->bound) return set_err(ctx, EDHMC_ESTATE, "no model bound");
   if (!W || !logp_out) return set_err(ctx, EDHMC_EINVAL, "NULL argument");
-  EDHMC_TRY(ensure_chains(ctx, C));
+  EDHMC_TRY(ensure_chains(ctx, C, st));
   EDHMC_TRY(dev_alloc(ctx, ctx->tmp_count, 4));
   ChainArgs a = chain_args(ctx);
   a.W_in = W;
@@ -2293,7 +2397,7 @@ int edhmc_predict(edhmc_ctx* ctx, const float* W, int32_t S, float* mean_out, do
   hipStream_t st = (hipStream_t)stream;
   if (!ctx->bound) return set_err(ctx, EDHMC_ESTATE, "no model bound");
   if (!W) return set_err(ctx, EDHMC_EINVAL, "W is NULL");
-  EDHMC_TRY(ensure_chains(ctx, S));
+  EDHMC_TRY(ensure_chains(ctx, S, st));
   EDHMC_TRY(dev_alloc(ctx, ctx->tmp_count, 4));
   ChainArgs a = chain_args(ctx);
   a.W_in = W;
@@ -2344,8 +2448,7 @@ static int sg_step(edhmc_ctx* ctx, bool hamiltonian, float lr, float friction, f
     EDHMC_TRY(glm_write_lp(ctx, st));
     EDHMC_TRY(grad_eval(ctx, true, true, st));
     ChainArgs e = chain_args(ctx);
-    hipLaunchKernelGGL(chain_eval_kernel, dim3(ctx->C), dim3(kChainThreads), 0, st, e);
-    EDHMC_TRY(check_launch(ctx, "chain_eval"));
+    EDHMC_TRY(launch_chain(ctx, kChainEval, e, st));
   }
   surrogate_invalidate(ctx->sur);
   ChainArgs a = chain_args(ctx);

@@ -30,7 +30,7 @@ namespace edhmc {
 
 int glm_grad_eval_offset(edhmc_ctx* ctx, const float* goff, int64_t goff_ld, const int* gidx,
                          bool ll, hipStream_t st);
-int glm_ensure_chains(edhmc_ctx* ctx, int C);
+int glm_ensure_chains(edhmc_ctx* ctx, int C, hipStream_t st);
 
 struct HierModel {
   int G = 0, D = 0, dim = 0, dim_pad = 0;
@@ -340,7 +340,7 @@ static int hier_set_state(edhmc_ctx* ctx, const float* theta, int C, hipStream_t
   HierModel* h = ctx->hier;
   if (!h) return set_err(ctx, EDHMC_ESTATE, "no hierarchical model bound");
   if (!theta) return set_err(ctx, EDHMC_EINVAL, "theta is NULL");
-  EDHMC_TRY(glm_ensure_chains(ctx, C));
+  EDHMC_TRY(glm_ensure_chains(ctx, C, st));
   if (h->C != C || h->C_pad != ctx->C_pad) {
     const size_t b = (size_t)ctx->C_pad * h->dim_pad * 4;
     EDHMC_TRY(dev_alloc(ctx, h->th, b));
