@@ -117,6 +117,7 @@ struct edhmc_ctx {
   edhmc::DevBuf pred_col;   // posterior-predictive column partials [m_tiles][N_pad]
   edhmc::DevBuf ll_split;   // log-likelihood range sums [16][C_pad] (fixed-order reduction)
   edhmc::DevBuf newton;          // scratch of edhmc_newton_terms
+  edhmc::DevBuf acov_part, acov_mean;   // autocovariance partial sums, chain means
 
   edhmc::Profiler prof;
   edhmc::Surrogate* sur = nullptr;
@@ -154,6 +155,12 @@ inline int dev_alloc(edhmc_ctx* ctx, DevBuf& b, size_t bytes, bool zero = true) 
   if (zero && hipMemset(b.p, 0, bytes) != hipSuccess)
     return set_err(ctx, EDHMC_EHIP, "hipMemset failed");
   return EDHMC_OK;
+}
+
+// At least `bytes`, contents undefined; grows only (scratch whose size varies
+// from call to call).
+inline int dev_reserve(edhmc_ctx* ctx, DevBuf& b, size_t bytes) {
+  return b.p && b.bytes >= bytes ? EDHMC_OK : dev_alloc(ctx, b, bytes, false);
 }
 
 // Bracket a launch with profiler events when profiling is on.

@@ -944,45 +944,6 @@ __global__ void rng_uniforms_kernel(int C, uint64_t seed, uint64_t counter, doub
   if (c < C) out[c] = accept_uniform(seed, counter, (uint32_t)c);
 }
 
-// Autocovariance for ESS: thread per (chain, coordinate); lags in blocks of 16
-// with a register window.
-__global__ void __launch_bounds__(256)
-autocov_kernel(const float* __restrict__ s, int64_t T, int C, int D, int max_lag,
-               double* __restrict__ acov, double* __restrict__ cmean) {
-  const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (id >= (int64_t)C * D) return;
-  const int c = (int)(id / D), d = (int)(id - (int64_t)c * D);
-  const int64_t stride = (int64_t)C * D;
-  const float* x = s + (int64_t)c * D + d;
-  double m = 0.0;
-  for (int64_t i = 0; i < T; ++i) m += x[i * stride];
-  m /= (double)T;
-  if (cmean) cmean[id] = m;
-  for (int l0 = 0; l0 <= max_lag; l0 += 16) {
-    double acc[16];
-    float win[16];
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      acc[k] = 0.0;
-      const int64_t j = l0 + k;
-      win[k] = j < T ? x[j * stride] : 0.0f;
-    }
-    for (int64_t i = 0; i + l0 < T; ++i) {
-      const double xi = (double)x[i * stride] - m;
-#pragma unroll
-      for (int k = 0; k < 16; ++k)
-        if (i + l0 + k < T) acc[k] += xi * ((double)win[k] - m);
-#pragma unroll
-      for (int k = 0; k < 15; ++k) win[k] = win[k + 1];
-      const int64_t j = i + l0 + 16;
-      win[15] = j < T ? x[j * stride] : 0.0f;
-    }
-#pragma unroll
-    for (int k = 0; k < 16; ++k)
-      if (l0 + k <= max_lag) atomicAdd(&acov[(int64_t)(l0 + k) * D + d], acc[k] / (double)T);
-  }
-}
-
 // Column statistics, pass 1: per (row chunk, column) FP64 sum and sum of
 // squares; pass 2: fixed-order combination.
 __global__ void __launch_bounds__(256)
@@ -1017,26 +978,6 @@ __global__ void col_stats_final_kernel(const double* __restrict__ part, int64_t 
   const double v = fmax(q / (double)P - m * m, 0.0);
   mean[d] = (float)m;
   sd[d] = (float)sqrt(v);
-}
-
-// Empirical moments: thread per column, two passes over rows t0..T-1.
-template <typename P>
-__global__ void __launch_bounds__(256)
-sample_moments_kernel(const P* __restrict__ x, int64_t T, int64_t K, int64_t t0,
-                      double* __restrict__ mean, double* __restrict__ var) {
-  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= K) return;
-  double s = 0.0;
-  for (int64_t t = t0; t < T; ++t) s += (double)x[t * K + k];
-  const double n = (double)(T - t0);
-  const double m = s / n;
-  double q = 0.0;
-  for (int64_t t = t0; t < T; ++t) {
-    const double d = (double)x[t * K + k] - m;
-    q += d * d;
-  }
-  mean[k] = m;
-  var[k] = q / n;
 }
 
 // ---------------------------------------------------------------------------
@@ -2198,7 +2139,7 @@ edhmc_ctx::~edhmc_ctx() {
   DevBuf* bufs[] = {&Xr, &Xc, &Xf, &Xs, &y, &ploc, &pscale, &z, &r, &g, &z0, &g0, &z_lp, &logp, &K0,
                     &flag, &ndiv, &ratio, &Rt, &Gpart, &llpart, &ll, &mom_mean, &mom_m2, &tmp_count,
                     &stats_part, &pred_col, &ll_split, &pkind, &plnorm,
-                    &newton};
+                    &newton, &acov_part, &acov_mean};
   for (DevBuf* b : bufs) b->release();
 }
 
@@ -2805,26 +2746,6 @@ int edhmc_draw_uniforms(edhmc_ctx* ctx, int32_t C, uint64_t seed, uint64_t count
   return check_launch(ctx, "rng_uniforms");
 }
 
-int edhmc_sample_moments(edhmc_ctx* ctx, const void* params, int32_t params_dtype, int64_t T,
-                         int64_t K, int64_t t0, double* mean_out, double* var_out, void* stream) {
-  if (!ctx) return EDHMC_EINVAL;
-  DeviceGuard dg(ctx->device);
-  if (!params || !mean_out || !var_out || T <= 0 || K <= 0 || t0 < 0 || t0 >= T)
-    return set_err(ctx, EDHMC_EINVAL, "bad arguments (T=%lld K=%lld t0=%lld)", (long long)T,
-                   (long long)K, (long long)t0);
-  if (params_dtype != EDHMC_F32 && params_dtype != 2)
-    return set_err(ctx, EDHMC_EINVAL, "params dtype must be fp32 or fp64");
-  hipStream_t st = (hipStream_t)stream;
-  const unsigned blocks = (unsigned)((K + 255) / 256);
-  if (params_dtype == EDHMC_F32)
-    hipLaunchKernelGGL(sample_moments_kernel<float>, dim3(blocks), dim3(256), 0, st,
-                       (const float*)params, T, K, t0, mean_out, var_out);
-  else
-    hipLaunchKernelGGL(sample_moments_kernel<double>, dim3(blocks), dim3(256), 0, st,
-                       (const double*)params, T, K, t0, mean_out, var_out);
-  return check_launch(ctx, "sample_moments");
-}
-
 int edhmc_record_pairs(edhmc_ctx* ctx, float* W_buf, float* G_buf, int64_t capacity,
                        int32_t stride) {
   if (!ctx) return EDHMC_EINVAL;
@@ -2869,22 +2790,6 @@ int edhmc_col_stats_noalloc(edhmc_ctx* ctx, const float* X, int64_t P, int32_t D
   // pass of this call: nothing needs clearing
   const int chunks = (int)std::min<int64_t>(kStatsChunks, P);
   return col_stats_launch(ctx, X, P, D, chunks, part, mean_out, std_out, (hipStream_t)stream);
-}
-
-int edhmc_autocov(edhmc_ctx* ctx, const float* s, int64_t T, int32_t C, int32_t D, int32_t max_lag,
-                  double* acov_out, double* chain_mean_out, void* stream) {
-  if (!ctx) return EDHMC_EINVAL;
-  DeviceGuard dg(ctx->device);
-  hipStream_t st = (hipStream_t)stream;
-  if (!s || !acov_out || T < 2 || C <= 0 || D <= 0 || max_lag < 0)
-    return set_err(ctx, EDHMC_EINVAL, "bad arguments");
-  if (max_lag >= T) max_lag = (int)(T - 1);
-  if (hipMemsetAsync(acov_out, 0, (size_t)(max_lag + 1) * D * 8, st) != hipSuccess)
-    return set_err(ctx, EDHMC_EHIP, "memset failed");
-  const int64_t n = (int64_t)C * D;
-  hipLaunchKernelGGL(autocov_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, s, T, C,
-                     D, max_lag, acov_out, chain_mean_out);
-  return check_launch(ctx, "autocov");
 }
 
 }  // extern "C"

@@ -32,57 +32,72 @@ def autocov(engine, samples, max_lag):
   return acov, cmean
 
 
+def autocov_lags(engine, samples, lag0, n_lags, chain_means):
+  """The sums of :func:`autocov` at lags lag0 .. lag0 + n_lags - 1 only,
+  [n_lags, D] fp64, from the chain means it returned."""
+  s = samples.contiguous()
+  T, C, D = s.shape
+  acov = torch.empty(n_lags, D, dtype=torch.float64, device=s.device)
+  engine.check(engine.lib.edhmc_autocov_lags(engine.h, L.ptr(s), T, C, D, int(lag0), int(n_lags),
+                                             L.ptr(chain_means), L.ptr(acov), engine.stream))
+  return acov
+
+
 def ess_from_acov(acov_sum, chain_means, n, between=False):
   """ESS per coordinate from summed autocovariances [lags, D] and chain means
   [M, D] of n draws per chain."""
-  acov_sum = np.asarray(acov_sum, np.float64)
   chain_means = np.asarray(chain_means, np.float64)
-  M, D = chain_means.shape
-  lags = acov_sum.shape[0]
+  M = chain_means.shape[0]
+  spread = chain_means.var(axis=0, ddof=1) if between and M > 1 else 0.0
+  return _ess_from_spread(np.asarray(acov_sum, np.float64), spread, M, n)
+
+
+def _ess_from_spread(acov_sum, spread, M, n):
+  """:func:`ess_from_acov` from the variance of the chain means over the
+  chains (0 where the spread is left out)."""
+  lags, D = acov_sum.shape
   acov_mean = acov_sum / M
   W = acov_mean[0] * n / (n - 1.0)
-  var_plus = W * (n - 1.0) / n
-  if between and M > 1:
-    var_plus = var_plus + chain_means.var(axis=0, ddof=1)
-  out = np.empty(D)
-  for d in range(D):
-    if not var_plus[d] > 0:
-      out[d] = 0.0            # no movement: nothing was sampled
-      continue
-    rho = 1.0 - (W[d] - acov_mean[:, d]) / var_plus[d]
-    rho[0] = 1.0
-    total, prev, k = 0.0, float('inf'), 0
-    truncated = False
-    while 2 * k + 1 < lags:
-      p = rho[2 * k] + rho[2 * k + 1]
-      if p <= 0:
-        truncated = True
-        break
-      p = min(p, prev)
-      total += p
-      prev = p
-      k += 1
-    if not truncated and 2 * k + 1 >= lags and lags < n:
-      out[d] = float('nan')      # lag window too short: caller widens it
-      continue
-    tau = max(-1.0 + 2.0 * total, 1.0 / math.log10(M * n))
-    out[d] = M * n / tau
+  var_plus = W * (n - 1.0) / n + spread
+  moved = var_plus > 0               # no movement: nothing was sampled
+  rho = 1.0 - (W - acov_mean) / np.where(moved, var_plus, 1.0)
+  rho[0] = 1.0
+  pairs = lags // 2
+  p = rho[0:2 * pairs:2] + rho[1:2 * pairs:2]
+  # Geyer's initial sequence: the pairs before the first that is not
+  # positive, made non-increasing
+  stop = np.concatenate([p <= 0, np.ones((1, D), bool)])
+  k = stop.argmax(axis=0)
+  truncated = k < pairs
+  total = np.zeros((pairs + 1, D))
+  np.cumsum(np.minimum.accumulate(p, axis=0), axis=0, out=total[1:])
+  tau = np.maximum(-1.0 + 2.0 * total[k, np.arange(D)], 1.0 / math.log10(M * n))
+  out = np.where(moved, M * n / tau, 0.0)
+  if lags < n:                       # lag window too short: caller widens it
+    out[moved & ~truncated] = np.nan
   return out
 
 
 def ess(engine, samples, max_lag=64, between=True):
   """Per-coordinate ESS of samples [T, C, D] (device, fp32); the lag window
-  doubles until every coordinate's Geyer sequence is truncated."""
-  T = samples.shape[0]
+  doubles until every coordinate's Geyer sequence is truncated (each lag is
+  summed once)."""
+  T, M, D = (int(v) for v in samples.shape)
   if T < 4:
-    return np.full(int(samples.shape[2]), np.nan)   # too few draws to estimate
+    return np.full(D, np.nan)   # too few draws to estimate
+  s = samples.contiguous()
   lag = min(max_lag, T - 1)
+  acov, cmean = autocov(engine, s, lag)
+  acov = acov.cpu().numpy()
+  spread = cmean.cpu().numpy().var(axis=0, ddof=1) if between and M > 1 else 0.0
   while True:
-    acov, cmean = autocov(engine, samples, lag)
-    e = ess_from_acov(acov.cpu().numpy(), cmean.cpu().numpy(), T, between=between)
+    e = _ess_from_spread(acov, spread, M, T)
     if not np.any(np.isnan(e)) or lag >= T - 1:
       return np.where(np.isnan(e), 0.0, e)
-    lag = min(2 * lag + 1, T - 1)
+    wider = min(2 * lag + 1, T - 1)
+    more = autocov_lags(engine, s, lag + 1, wider - lag, cmean)
+    acov = np.concatenate([acov, more.cpu().numpy()])
+    lag = wider
 
 
 def min_ess(engine, samples, max_lag=64, between=True):

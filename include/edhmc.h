@@ -329,6 +329,13 @@ int edhmc_draw_uniforms(edhmc_ctx* ctx, int32_t C, uint64_t seed, uint64_t count
 int edhmc_autocov(edhmc_ctx* ctx, const float* s, int64_t T, int32_t C, int32_t D,
                   int32_t max_lag, double* acov_out, double* chain_mean_out,
                   void* stream);
+/* The same autocovariances at lags lag0 .. lag0 + n_lags - 1 only
+ * (lag0 + n_lags <= T), acov_out [n_lags, D] fp64, from the chain means
+ * [C, D] fp64 that edhmc_autocov wrote for the same store: a window that
+ * turns out too short is widened without its lags a second time. */
+int edhmc_autocov_lags(edhmc_ctx* ctx, const float* s, int64_t T, int32_t C, int32_t D,
+                       int32_t lag0, int32_t n_lags, const double* chain_mean,
+                       double* acov_out, void* stream);
 
 /* ------------------------------------------------------------------------
  * Learned gradient surrogate (no reference counterpart; build-only).
