@@ -48,6 +48,20 @@ struct Profiler {
   }
 };
 
+// What the gradient pass of the hierarchical model needs beside the GLM's:
+// intercepts goff[c * goff_ld + g], the group of each row (gidxp: in
+// grad_rows.h's row order), the groups' row offsets, and where their residual
+// sums go (ga[c * G + g]).
+struct HierRows {
+  const float* goff = nullptr;
+  int64_t goff_ld = 0;
+  const int* gidx = nullptr;
+  const int* gidxp = nullptr;
+  const int64_t* off = nullptr;
+  float* ga = nullptr;
+  int G = 0;
+};
+
 // A device allocation owned by the context, or (view) a part of another one.
 struct DevBuf {
   void* p = nullptr;
@@ -86,6 +100,8 @@ struct edhmc_ctx {
   int D = 0, D_pad = 0;
   edhmc::DevBuf Xr, Xc, y, ploc, pscale;
   edhmc::DevBuf Xf;   // bf16 X in MFMA fragment order (the W-stationary kernels' copy)
+  edhmc::DevBuf Xp, yp;   // fp32, D_pad <= 256: permuted copies for the one-pass gradient
+                          // (then there is no Xc)
   edhmc::DevBuf pkind, plnorm;   // constrained prior families (has_kinds)
   bool has_kinds = false;
 

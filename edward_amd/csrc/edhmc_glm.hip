@@ -10,7 +10,9 @@
 //          leapfrog kick/drift -- or, after the last step, the Metropolis
 //          test of hmc.py:100-111 and the sample write of hmc.py:121-129.
 // X is stored twice, row-major Xr [N, D] (GEMM1's B) and column-major
-// Xc [D, N] (GEMM2's B), so every MFMA operand is K-contiguous.
+// Xc [D, N] (GEMM2's B), so every MFMA operand is K-contiguous.  In fp32 with
+// D_pad <= 256 one kernel does both products (grad_rows.h; up to four chains:
+// few_chains.h) and the second copy is its permuted X.
 #include <algorithm>
 #include <cmath>
 #include <mutex>
@@ -21,6 +23,7 @@
 #include "gemm_nt.h"
 #include "gemm2_dma.h"
 #include "few_chains.h"
+#include "grad_rows.h"
 #include "philox.h"
 #include "transform.h"
 
@@ -376,13 +379,15 @@ colsum_reduce_kernel(const float* __restrict__ part, int m_tiles, int64_t ld, in
 }
 
 // ---------------------------------------------------------------------------
-// Data layout: X [N, D] (fp32 or bf16 in) -> Xr [N_pad, D_pad], Xc [D_pad, N_pad]
-// in the compute type; counts non-finite inputs.
+// Data layout: X [N, D] (fp32 or bf16 in) -> Xr [N_pad, D_pad] and either Xc
+// [D_pad, N_pad] or Xp (grad_rows.h), in the compute type; counts non-finite
+// inputs.
 // ---------------------------------------------------------------------------
 template <typename Tin, typename T>
 __global__ void __launch_bounds__(256)
 layout_x_kernel(const Tin* __restrict__ X, int64_t N, int D, T* __restrict__ Xr,
-                T* __restrict__ Xc, int64_t N_pad, int D_pad, int* nonfinite) {
+                T* __restrict__ Xc, T* __restrict__ Xp, int64_t N_pad, int D_pad,
+                int* nonfinite) {
   __shared__ float tile[32][33];
   const int64_t n0 = (int64_t)blockIdx.y * 32;
   const int d0 = blockIdx.x * 32;
@@ -399,8 +404,11 @@ layout_x_kernel(const Tin* __restrict__ X, int64_t N, int D, T* __restrict__ Xr,
     }
     tile[k][tx] = v;
     Xr[n * D_pad + d] = ElemOps<T>::from_f32(v);
+    // the one-pass gradient's copy: columns of every 16 in pi order
+    if (Xp) Xp[n * D_pad + (d & ~15) + pi16_inv(d & 15)] = ElemOps<T>::from_f32(v);
   }
   if (bad) atomicAdd(nonfinite, 1);
+  if (!Xc) return;   // uniform over the grid
   __syncthreads();
   // Xc is K-blocked: [N_pad / KE][D_pad][KE] with KE = 64 bytes of T.
   constexpr int KE = kStageBytes / sizeof(T);
@@ -592,6 +600,7 @@ __global__ void __launch_bounds__(kChainThreads) chain_begin_kernel(ChainArgs a)
 __device__ inline float gsum(const ChainArgs& a, int c, int d) {
   const float* p = a.Gpart + (int64_t)c * a.D_pad + d;
   float s = 0.0f;
+#pragma unroll 16
   for (int q = 0; q < a.ksplit; ++q) s += p[q * a.g_stride];
   return a.lik_weight * s;
 }
@@ -1192,7 +1201,48 @@ static int few_eval(edhmc_ctx* ctx, bool grad, bool ll, hipStream_t st) {
   return ll ? ll_reduce(ctx, a.splits, st) : EDHMC_OK;
 }
 
+// One-pass gradient with the two GEMMs' summation order (grad_rows.h); hr: the
+// hierarchical model's, whose residuals go to Rt, or with *summed set are
+// summed over the groups that lie within a range of that many rows and kept
+// in Rt for the other groups only.
+static int rows_eval(edhmc_ctx* ctx, bool ll, hipStream_t st, const HierRows* hr = nullptr,
+                     int64_t* summed = nullptr) {
+  RowsArgs a = {};
+  a.Xp = (const float*)ctx->Xp.p;
+  a.yp = (const float*)ctx->yp.p;
+  a.W = (const float*)ctx->z_lp.p;
+  a.N = ctx->N;
+  a.N_pad = ctx->N_pad;
+  const int64_t stages = ctx->N_pad * 4 / kStageBytes;
+  a.rows_per_split = (stages + ctx->ksplit - 1) / ctx->ksplit * (kStageBytes / 4);
+  a.C = ctx->C;
+  a.splits = ctx->ksplit;
+  a.lp = lik_params(ctx);
+  a.Gpart = (float*)ctx->Gpart.p;
+  a.g_ld = ctx->g_ld;
+  a.llpart = (double*)ctx->llpart.p;
+  a.ll_ld = ctx->C_pad;
+  if (hr) {
+    a.goff = hr->goff;
+    a.goff_ld = hr->goff_ld;
+    a.gidx = hr->gidx;
+    a.gidxp = hr->gidxp;
+    a.off = hr->off;
+    a.ga = hr->ga;
+    a.G = hr->G;
+    a.Rt = (float*)ctx->Rt.p;
+    a.ldr = ctx->C_pad;
+    *summed = rows_wide(a.C, a.splits) ? a.rows_per_split : 0;
+  }
+  {
+    ProfScope ps(ctx, PK_GEMM_GRAD, st);
+    EDHMC_TRY(rows_launch(ctx, a, ll, st));
+  }
+  return ll ? ll_reduce(ctx, a.splits, st) : EDHMC_OK;
+}
+
 static int grad_eval(edhmc_ctx* ctx, bool split, bool ll, hipStream_t st) {
+  if (rows_ok(ctx) && !ctx->few.on) return rows_eval(ctx, ll, st);
   if (ctx->few.on) return few_eval(ctx, true, ll, st);
   if (ctx->cdt == EDHMC_BF16) {
     if (split) {
@@ -1223,18 +1273,25 @@ static int grad_eval(edhmc_ctx* ctx, bool split, bool ll, hipStream_t st) {
 #ifndef EDHMC_CFG_H
 #define EDHMC_CFG_H 2, 2, 2, 2, 128
 #endif
-// GEMM1 of the hierarchical model (fp32, short K): 128-byte K stages halve
-// the stage barriers of its 2-4 stages (1.11 vs 1.19 ms per pass at G = 2048,
-// D = 64, 512 chains; 128 x 256 or 256 x 128 tiles leave one workgroup per
-// CU for the residual tile's LDS: 3.4-3.9 ms)
+// GEMM1 of the hierarchical model (its log-likelihood, and its residuals
+// where D_pad > 256): 128-byte K stages, half the stage barriers (1.11 vs
+// 1.19 ms at G = 2048, D = 64, 512 chains)
 using CfgH = TileCfg<EDHMC_CFG_H>;
-int glm_grad_eval_offset(edhmc_ctx* ctx, const float* goff, int64_t goff_ld, const int* gidx,
-                         bool ll, hipStream_t st) {
+int glm_grad_eval_offset(edhmc_ctx* ctx, const HierRows& hr, bool ll, hipStream_t st,
+                         int64_t* summed_rows) {
+  *summed_rows = 0;
   if (ctx->cdt != EDHMC_F32) return set_err(ctx, EDHMC_EUNSUPPORTED, "offset path is fp32");
+  if (rows_ok(ctx)) {
+    EDHMC_TRY(rows_eval(ctx, false, st, &hr, summed_rows));
+    // the log-likelihood in GEMM1's forward form: its FP64 partial sums keep
+    // their order over the rows
+    return ll ? launch_gemm1<float, CfgH, 1, false, true>(ctx, st, hr.goff, hr.goff_ld, hr.gidx)
+              : EDHMC_OK;
+  }
   if (ctx->C_pad % CfgH::BM || ctx->N_pad % CfgH::BN)
     return set_err(ctx, EDHMC_EUNSUPPORTED, "hierarchical GEMM1 tiles do not divide the padding");
-  if (ll) EDHMC_TRY((launch_gemm1<float, CfgH, 1, true, true>(ctx, st, goff, goff_ld, gidx)));
-  else EDHMC_TRY((launch_gemm1<float, CfgH, 1, true, false>(ctx, st, goff, goff_ld, gidx)));
+  if (ll) EDHMC_TRY((launch_gemm1<float, CfgH, 1, true, true>(ctx, st, hr.goff, hr.goff_ld, hr.gidx)));
+  else EDHMC_TRY((launch_gemm1<float, CfgH, 1, true, false>(ctx, st, hr.goff, hr.goff_ld, hr.gidx)));
   return launch_gemm2<float>(ctx, st);
 }
 
@@ -1982,9 +2039,11 @@ static int ensure_chains(edhmc_ctx* ctx, int C, hipStream_t st) {
                            (float*)ctx->Xs.p, st));
     }
   } else {
-    // rows up to a whole W-stationary tile: its residual epilogue stores the
+    // residuals: none after a one-pass gradient but the hierarchical model's;
+    // rows up to a whole W-stationary tile, whose residual epilogue stores the
     // last tile's rows past N_pad (zeros) without a bounds test
-    EDHMC_TRY(dev_alloc(ctx, ctx->Rt, (size_t)C_pad * round_up(ctx->N_pad, kWsTile) * eb, false));
+    if (rows_ok(ctx) && !ctx->hier) ctx->Rt.release();
+    else EDHMC_TRY(dev_alloc(ctx, ctx->Rt, (size_t)C_pad * round_up(ctx->N_pad, kWsTile) * eb, false));
     // split-K for GEMM2: aim for >= 2048 workgroups, >= 8 stages per split.
     const int bn2 = (ctx->D_pad % Cfg1::BN == 0) ? Cfg1::BN : Cfg2S::BN;
     const int tiles2 = (C_pad / 128) * (ctx->D_pad / bn2);
@@ -1994,6 +2053,7 @@ static int ensure_chains(edhmc_ctx* ctx, int C, hipStream_t st) {
     if (ks >= 8) ks = ks / 8 * 8;
     ctx->ksplit = ks;
     ctx->g_ld = C_pad;
+    ctx->n_tiles1 = std::max(ctx->n_tiles1, ks);   // one-pass gradient: partials per range
   }
   EDHMC_TRY(dev_alloc(ctx, ctx->Gpart, (size_t)ctx->ksplit * ctx->g_ld * ctx->D_pad * 4, false));
   EDHMC_TRY(dev_alloc(ctx, ctx->llpart, (size_t)C_pad * ctx->n_tiles1 * 8, false));
@@ -2136,7 +2196,7 @@ edhmc_ctx::~edhmc_ctx() {
   for (hipEvent_t e : prof.pool) (void)hipEventDestroy(e);
   if (sur) surrogate_destroy(sur);
   if (hier) hier_destroy(hier);
-  DevBuf* bufs[] = {&Xr, &Xc, &Xf, &Xs, &y, &ploc, &pscale, &z, &r, &g, &z0, &g0, &z_lp, &logp, &K0,
+  DevBuf* bufs[] = {&Xr, &Xc, &Xf, &Xs, &Xp, &yp, &y, &ploc, &pscale, &z, &r, &g, &z0, &g0, &z_lp, &logp, &K0,
                     &flag, &ndiv, &ratio, &Rt, &Gpart, &llpart, &ll, &mom_mean, &mom_m2, &tmp_count,
                     &stats_part, &pred_col, &ll_split, &pkind, &plnorm,
                     &newton, &acov_part, &acov_mean};
@@ -2206,7 +2266,15 @@ int edhmc_bind_glm(edhmc_ctx* ctx, const void* X, int32_t x_in_dtype, const floa
   ctx->D_pad = (int)round_up(D, 64);   // K of GEMM1 in whole 128-byte stages
   const int eb = elem_bytes(ctx);
   EDHMC_TRY(dev_alloc(ctx, ctx->Xr, (size_t)ctx->N_pad * ctx->D_pad * eb, false));
-  EDHMC_TRY(dev_alloc(ctx, ctx->Xc, (size_t)ctx->N_pad * ctx->D_pad * eb, false));
+  if (rows_ok(ctx)) {
+    ctx->Xc.release();
+    EDHMC_TRY(dev_alloc(ctx, ctx->Xp, (size_t)ctx->N_pad * ctx->D_pad * eb, false));
+    EDHMC_TRY(dev_alloc(ctx, ctx->yp, (size_t)ctx->N_pad * 4, false));
+  } else {
+    ctx->Xp.release();
+    ctx->yp.release();
+    EDHMC_TRY(dev_alloc(ctx, ctx->Xc, (size_t)ctx->N_pad * ctx->D_pad * eb, false));
+  }
   EDHMC_TRY(dev_alloc(ctx, ctx->y, (size_t)ctx->N_pad * 4, false));
   EDHMC_TRY(dev_alloc(ctx, ctx->ploc, (size_t)ctx->D_pad * 4, false));
   EDHMC_TRY(dev_alloc(ctx, ctx->pscale, (size_t)ctx->D_pad * 4, false));
@@ -2214,23 +2282,18 @@ int edhmc_bind_glm(edhmc_ctx* ctx, const void* X, int32_t x_in_dtype, const floa
   int* bad = (int*)ctx->tmp_count.p;
   dim3 grid(ctx->D_pad / 32, (unsigned)(ctx->N_pad / 32));
   if (ctx->N_pad / 32 > 2147483647LL) return set_err(ctx, EDHMC_EUNSUPPORTED, "N too large");
+  auto layout = [&](auto tin, auto t) {
+    using Tin = decltype(tin);
+    using T = decltype(t);
+    hipLaunchKernelGGL((layout_x_kernel<Tin, T>), grid, dim3(256), 0, st, (const Tin*)X, N, D,
+                       (T*)ctx->Xr.p, (T*)ctx->Xc.p, (T*)ctx->Xp.p, ctx->N_pad, ctx->D_pad, bad);
+  };
   if (x_in_dtype == EDHMC_F32) {
-    if (compute_dtype == EDHMC_F32)
-      hipLaunchKernelGGL((layout_x_kernel<float, float>), grid, dim3(256), 0, st, (const float*)X,
-                         N, D, (float*)ctx->Xr.p, (float*)ctx->Xc.p, ctx->N_pad, ctx->D_pad, bad);
-    else
-      hipLaunchKernelGGL((layout_x_kernel<float, bf16_t>), grid, dim3(256), 0, st,
-                         (const float*)X, N, D, (bf16_t*)ctx->Xr.p, (bf16_t*)ctx->Xc.p,
-                         ctx->N_pad, ctx->D_pad, bad);
+    if (compute_dtype == EDHMC_F32) layout(float{}, float{});
+    else layout(float{}, bf16_t{});
   } else {
-    if (compute_dtype == EDHMC_F32)
-      hipLaunchKernelGGL((layout_x_kernel<bf16_t, float>), grid, dim3(256), 0, st,
-                         (const bf16_t*)X, N, D, (float*)ctx->Xr.p, (float*)ctx->Xc.p,
-                         ctx->N_pad, ctx->D_pad, bad);
-    else
-      hipLaunchKernelGGL((layout_x_kernel<bf16_t, bf16_t>), grid, dim3(256), 0, st,
-                         (const bf16_t*)X, N, D, (bf16_t*)ctx->Xr.p, (bf16_t*)ctx->Xc.p,
-                         ctx->N_pad, ctx->D_pad, bad);
+    if (compute_dtype == EDHMC_F32) layout(bf16_t{}, float{});
+    else layout(bf16_t{}, bf16_t{});
   }
   EDHMC_TRY(check_launch(ctx, "layout_x"));
   ctx->Xf.release();
@@ -2247,6 +2310,7 @@ int edhmc_bind_glm(edhmc_ctx* ctx, const void* X, int32_t x_in_dtype, const floa
     return check_launch(ctx, "pad_copy");
   };
   EDHMC_TRY(padc(y, N, ctx->y, ctx->N_pad, 0.0f));
+  if (ctx->yp.p) EDHMC_TRY(rows_permute(ctx, ctx->y.p, ctx->N_pad, ctx->yp.p, st));
   EDHMC_TRY(padc(prior_loc, D, ctx->ploc, ctx->D_pad, 0.0f));
   EDHMC_TRY(padc(prior_scale, D, ctx->pscale, ctx->D_pad, 1.0f));
   int nbad = 0;

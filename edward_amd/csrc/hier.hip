@@ -28,8 +28,9 @@
 
 namespace edhmc {
 
-int glm_grad_eval_offset(edhmc_ctx* ctx, const float* goff, int64_t goff_ld, const int* gidx,
-                         bool ll, hipStream_t st);
+int glm_grad_eval_offset(edhmc_ctx* ctx, const HierRows& hr, bool ll, hipStream_t st,
+                         int64_t* summed_rows);
+int rows_permute(edhmc_ctx* ctx, const void* in, int64_t n, void* out, hipStream_t st);
 int glm_ensure_chains(edhmc_ctx* ctx, int C, hipStream_t st);
 
 struct HierModel {
@@ -40,7 +41,7 @@ struct HierModel {
   float sp1 = 0.0f, sp2 = 1.0f;
   double slnorm = -0.5 * kLog2Pi;
   int64_t N = 0;
-  DevBuf gidx, offsets, ones, zeros;
+  DevBuf gidx, gidxp, offsets, ones, zeros;   // gidx: group of each row; gidxp: in grad_rows.h's row order
   int C = 0, C_pad = 0;
   bool state_valid = false;
   DevBuf th, r, g, th0, g0, ga, logp, K0;
@@ -48,7 +49,7 @@ struct HierModel {
 
 void hier_destroy(HierModel* h) {
   if (!h) return;
-  DevBuf* b[] = {&h->gidx, &h->offsets, &h->ones, &h->zeros, &h->th, &h->r, &h->g, &h->th0,
+  DevBuf* b[] = {&h->gidx, &h->gidxp, &h->offsets, &h->ones, &h->zeros, &h->th, &h->r, &h->g, &h->th0,
                  &h->g0, &h->ga, &h->logp, &h->K0};
   for (DevBuf* x : b) x->release();
   delete h;
@@ -56,9 +57,11 @@ void hier_destroy(HierModel* h) {
 
 constexpr int kHT = 256;   // threads per chain workgroup
 
-__global__ void group_index_kernel(const int64_t* __restrict__ off, int G, int* __restrict__ gidx) {
+__global__ void group_index_kernel(const int64_t* __restrict__ off, int G, int64_t N_pad,
+                                   int* __restrict__ gidx) {
   const int g = blockIdx.x;
-  for (int64_t n = off[g] + threadIdx.x; n < off[g + 1]; n += blockDim.x) gidx[n] = g;
+  const int64_t e = g + 1 < G ? off[g + 1] : N_pad;   // the padding: the last group
+  for (int64_t n = off[g] + threadIdx.x; n < e; n += blockDim.x) gidx[n] = g;
 }
 
 // grad_a[c, g] = sum_{n in group g} R[c, n]; R^T is fp32 K-blocked
@@ -69,9 +72,11 @@ __global__ void group_index_kernel(const int64_t* __restrict__ off, int G, int* 
 // a fixed order (deterministic).
 __global__ void __launch_bounds__(256)
 seg_sum_kernel(const float* __restrict__ Rt, const int64_t* __restrict__ off, int C, int C_pad,
-               int G, float* __restrict__ ga) {
+               int G, int64_t summed, float* __restrict__ ga) {
   const int g = blockIdx.x;
   const int64_t b = off[g], e = off[g + 1];
+  // row ranges of `summed` rows (0: none) have summed the groups inside them
+  if (summed && e > b && b / summed == (e - 1) / summed) return;
   const int q = threadIdx.x & 3;
   const int64_t kb0 = b >> 4, kb1 = e > b ? ((e - 1) >> 4) : kb0 - 1;
   for (int c0 = 0; c0 < C; c0 += 64) {
@@ -160,6 +165,7 @@ __device__ inline void hier_assemble(const HierArgs& a, int c, bool want_lp, dou
       const int d = j - a.G - 2;
       const float* gp = a.Gpart + (int64_t)c * a.D_pad + d;
       float s = 0.0f;
+#pragma unroll 16
       for (int q = 0; q < a.ksplit; ++q) s += gp[q * gstride];
       gv = s - th[j];
     }
@@ -328,11 +334,20 @@ static HierArgs hier_args(edhmc_ctx* ctx, HierModel* h) {
 }
 
 static int hier_grad(edhmc_ctx* ctx, HierModel* h, bool ll, hipStream_t st) {
-  EDHMC_TRY(glm_grad_eval_offset(ctx, (const float*)h->th.p, h->dim_pad, (const int*)h->gidx.p,
-                                 ll, st));
+  HierRows hr;
+  hr.goff = (const float*)h->th.p;
+  hr.goff_ld = h->dim_pad;
+  hr.gidx = (const int*)h->gidx.p;
+  hr.gidxp = (const int*)h->gidxp.p;
+  hr.off = (const int64_t*)h->offsets.p;
+  hr.ga = (float*)h->ga.p;
+  hr.G = h->G;
+  int64_t summed = 0;
+  EDHMC_TRY(glm_grad_eval_offset(ctx, hr, ll, st, &summed));
   ProfScope ps(ctx, PK_HIER, st);
   hipLaunchKernelGGL(seg_sum_kernel, dim3(h->G), dim3(256), 0, st, (const float*)ctx->Rt.p,
-                     (const int64_t*)h->offsets.p, h->C, ctx->C_pad, h->G, (float*)h->ga.p);
+                     (const int64_t*)h->offsets.p, h->C, ctx->C_pad, h->G, summed,
+                     (float*)h->ga.p);
   return check_launch(ctx, "seg_sum");
 }
 
@@ -456,10 +471,12 @@ int edhmc_bind_hier(edhmc_ctx* ctx, const float* X, const float* y, const int64_
   if (hipMemcpyAsync(h->offsets.p, offsets, (size_t)(G + 1) * 8, hipMemcpyDeviceToDevice, st) !=
       hipSuccess)
     return set_err(ctx, EDHMC_EHIP, "copy offsets");
-  EDHMC_TRY(dev_alloc(ctx, h->gidx, (size_t)ctx->N_pad * 4));
+  EDHMC_TRY(dev_alloc(ctx, h->gidx, (size_t)ctx->N_pad * 4, false));
   hipLaunchKernelGGL(group_index_kernel, dim3(G), dim3(256), 0, st,
-                     (const int64_t*)h->offsets.p, G, (int*)h->gidx.p);
+                     (const int64_t*)h->offsets.p, G, ctx->N_pad, (int*)h->gidx.p);
   EDHMC_TRY(check_launch(ctx, "group_index"));
+  EDHMC_TRY(dev_alloc(ctx, h->gidxp, (size_t)ctx->N_pad * 4, false));
+  EDHMC_TRY(rows_permute(ctx, h->gidx.p, ctx->N_pad, h->gidxp.p, st));
   if (hipStreamSynchronize(st) != hipSuccess) return set_err(ctx, EDHMC_EHIP, "sync");
   return EDHMC_OK;
 }
