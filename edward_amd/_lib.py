@@ -91,6 +91,9 @@ SIGNATURES = {
     'edhmc_sur_train_step': (ctypes.c_int, [_c_p, _c_p, _c_p, _i32, _f32, _f32, _f32, _f32,
                                             _i32, _c_p, _c_p]),
     'edhmc_gather_rows': (ctypes.c_int, [_c_p, _c_p, _i64, _i32, _c_p, _i32, _c_p, _c_p]),
+    'edhmc_solve_spd_work': (_i64, [_i32]),
+    'edhmc_solve_spd': (ctypes.c_int, [_c_p, _c_p, _c_p, _i32, ctypes.c_double, _c_p, _c_p, _c_p,
+                                       _c_p]),
     'edhmc_sur_skip_gram': (ctypes.c_int, [_c_p, _c_p, _c_p, _i64, _c_p, _i32, _c_p, _c_p,
                                            _c_p]),
     'edhmc_affine_rows': (ctypes.c_int, [_c_p, _c_p, _i64, _i32, _c_p, _c_p, _c_p, _c_p]),

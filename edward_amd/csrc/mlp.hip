@@ -87,7 +87,13 @@ struct Surrogate {
   DevBuf ghat, ghat0;                  // [C x D_pad of the GLM]
   bool ghat_valid = false;
   bool norm_set = false;
+  DevBuf gram;                         // skip_gram's partial products
+  hipEvent_t gram_used = nullptr;
 };
+
+int skip_gram(edhmc_ctx* ctx, DevBuf& scratch, hipEvent_t& used, const float* W, const float* G,
+              int64_t P, int D, const int64_t* idx, int n, const float* nrm, int Dp, double* xtx,
+              double* xtt, hipStream_t st);
 
 void surrogate_invalidate(Surrogate* s) {
   if (s) s->ghat_valid = false;
@@ -98,8 +104,9 @@ void surrogate_destroy(Surrogate* s) {
   DevBuf* b[] = {&s->P, &s->Gr, &s->Am, &s->Av, &s->W1b, &s->W2b, &s->W3b, &s->W2t, &s->W3t,
                  &s->nrm, &s->x0, &s->a1, &s->h1, &s->a2, &s->h2, &s->h2x, &s->o, &s->dO, &s->da2,
                  &s->da1, &s->h1t, &s->h2t, &s->dOt, &s->da2t, &s->da1t, &s->loss,
-                 &s->lpart, &s->ghat, &s->ghat0, &s->pool};
+                 &s->lpart, &s->ghat, &s->ghat0, &s->pool, &s->gram};
   for (DevBuf* x : b) x->release();
+  if (s->gram_used) (void)hipEventDestroy(s->gram_used);
   delete s;
 }
 
@@ -483,66 +490,6 @@ __global__ void rowsum_bf16_kernel(const bf16_t* __restrict__ in, int R, int K, 
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
   if (lane == 0) out[row] = s;
-}
-
-// Least-squares Gram products of the output layer's linear skip over the
-// rows idx[0..n) of (W, G): x = (w - in_shift) * in_scale and t = (g -
-// out_shift) / out_scale in fp32, out = sum_rows x^T x (blockIdx.z = 0) or
-// x^T t (z = 1), [D x D] FP64.  A 64 x 64 output block per workgroup, a
-// thread owning 4 x 4 entries, rows staged 32 at a time through LDS.  An
-// index outside [0, P) contributes NaN.
-__global__ void __launch_bounds__(256)
-skip_gram_kernel(const float* __restrict__ W, const float* __restrict__ G, int64_t P, int D,
-                 const int64_t* __restrict__ idx, int n, const float* __restrict__ nrm, int Dp,
-                 double* __restrict__ xtx, double* __restrict__ xtt) {
-  __shared__ float la[32][64], lb[32][64];
-  const int i0 = blockIdx.y * 64, j0 = blockIdx.x * 64, z = blockIdx.z;
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  const float* in_shift = nrm;
-  const float* in_scale = nrm + Dp;
-  const float* out_shift = nrm + 2 * Dp;
-  const float* out_scale = nrm + 3 * Dp;
-  double acc[4][4] = {};
-  for (int r0 = 0; r0 < n; r0 += 32) {
-    for (int q = threadIdx.x; q < 32 * 64; q += 256) {
-      const int rr = q >> 6, c = q & 63, row = r0 + rr;
-      float a = 0.0f, b = 0.0f;
-      if (row < n && (idx[row] < 0 || idx[row] >= P)) {
-        a = b = __builtin_nanf("");
-      } else if (row < n) {
-        const int64_t src = idx[row] * (int64_t)D;
-        if (i0 + c < D) a = (W[src + i0 + c] - in_shift[i0 + c]) * in_scale[i0 + c];
-        const int j = j0 + c;
-        if (j < D) b = z == 0 ? (W[src + j] - in_shift[j]) * in_scale[j]
-                              : (G[src + j] - out_shift[j]) / out_scale[j];
-      }
-      la[rr][c] = a;
-      lb[rr][c] = b;
-    }
-    __syncthreads();
-#pragma unroll 4
-    for (int rr = 0; rr < 32; ++rr) {
-      float av[4], bv[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        av[u] = la[rr][ty * 4 + u];
-        bv[u] = lb[rr][tx * 4 + u];
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) acc[u][v] += (double)av[u] * (double)bv[v];
-    }
-    __syncthreads();
-  }
-  double* out = z == 0 ? xtx : xtt;
-#pragma unroll
-  for (int u = 0; u < 4; ++u)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int i = i0 + ty * 4 + u, j = j0 + tx * 4 + v;
-      if (i < D && j < D) out[(int64_t)i * D + j] = acc[u][v];
-    }
 }
 
 // out [n x D] = shift + E [n x D] R [D x D] (fp32; 64 x 64 output blocks, a
@@ -1354,10 +1301,8 @@ int edhmc_sur_skip_gram(edhmc_ctx* ctx, const float* W, const float* G, int64_t 
   if (!s->norm_set) return set_err(ctx, EDHMC_ESTATE, "normalisation not set");
   if (!W || !G || !idx || !xtx_out || !xtt_out || n <= 0 || P <= 0)
     return set_err(ctx, EDHMC_EINVAL, "bad arguments");
-  const int nb = (s->D + 63) / 64;
-  hipLaunchKernelGGL(skip_gram_kernel, dim3(nb, nb, 2), dim3(256), 0, (hipStream_t)stream, W, G,
-                     P, s->D, idx, n, (const float*)s->nrm.p, s->Dp, xtx_out, xtt_out);
-  return check_launch(ctx, "skip_gram");
+  return skip_gram(ctx, s->gram, s->gram_used, W, G, P, s->D, idx, n, (const float*)s->nrm.p, s->Dp,
+                   xtx_out, xtt_out, (hipStream_t)stream);
 }
 
 int edhmc_affine_rows(edhmc_ctx* ctx, const float* E, int64_t n, int32_t D, const float* R,

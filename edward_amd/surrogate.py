@@ -75,7 +75,8 @@ class Surrogate(object):
     """Start the output layer's linear skip at the least-squares map from the
     normalised inputs to the normalised targets, over an evenly spaced sample
     of ``rows`` (default all) of the pairs (W, G): the Gram products in FP64
-    on the device (``edhmc_sur_skip_gram``), the D x D solve on the host."""
+    and the D x D solve on the device (``edhmc_sur_skip_gram``,
+    ``edhmc_solve_spd``)."""
     eng = self.engine
     P = int(W.shape[0])
     rows = np.arange(P) if rows is None else np.asarray(rows, np.int64)
@@ -85,15 +86,21 @@ class Surrogate(object):
     xtt = torch.empty_like(xtx)
     eng.check(eng.lib.edhmc_sur_skip_gram(eng.h, L.ptr(W), L.ptr(G), P, L.ptr(idx), len(sel),
                                           L.ptr(xtx), L.ptr(xtt), eng.stream))
-    xtx = xtx.cpu().numpy()
-    xtt = xtt.cpu().numpy()
-    A = np.linalg.solve(xtx + ridge * len(sel) * np.eye(self.D), xtt)   # t ~ x A
-    # written into the device copy of the parameters (only the D x D block
-    # crosses to the device)
+    # t ~ x A: the positive definite solve on the device, A transposed
+    At = torch.empty(self.D, self.D, device=eng.device)
+    bad = torch.empty(1, dtype=torch.int32, device=eng.device)
+    work = torch.empty(eng.lib.edhmc_solve_spd_work(self.D), dtype=torch.uint8, device=eng.device)
+    eng.check(eng.lib.edhmc_solve_spd(eng.h, L.ptr(xtx), L.ptr(xtt), self.D,
+                                      float(ridge * len(sel)), L.ptr(At), L.ptr(bad),
+                                      L.ptr(work), eng.stream))
+    if int(bad.item()):   # a pivot <= 0 or NaN: the general solve, with its errors
+      A = np.linalg.solve(xtx.cpu().numpy() + ridge * len(sel) * np.eye(self.D),
+                          xtt.cpu().numpy())
+      At = torch.from_numpy(np.ascontiguousarray(A.T, dtype=np.float32)).to(eng.device)
     flat = self.get_params()
     o = self._offsets()
     W3 = flat[o['W3']:o['b3']].view(self.D, self.H + self.D)
-    W3[:, self.H:] = torch.from_numpy(np.ascontiguousarray(A.T, dtype=np.float32)).to(eng.device)
+    W3[:, self.H:] = At
     flat[o['b3']:o['b3'] + self.D] = 0.0
     self.set_params(flat)
     self.step_count = 0

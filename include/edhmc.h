@@ -402,6 +402,15 @@ int edhmc_sur_skip_gram(edhmc_ctx* ctx, const float* W, const float* G, int64_t 
                         const int64_t* idx, int32_t n, double* xtx_out, double* xtt_out,
                         void* stream);
 
+/* The solution X of (A + ridge I) X = B, A [n, n] symmetric positive definite
+ * and B [n, n] in fp64, transposed and rounded to fp32: xt_out[j][i] = X[i][j].
+ * *status (device) becomes 1 where a pivot of the elimination was not
+ * positive (X is then void), else 0.  work: edhmc_solve_spd_work(n) bytes of
+ * device memory.  No reference counterpart (the surrogate's linear skip). */
+int64_t edhmc_solve_spd_work(int32_t n);
+int edhmc_solve_spd(edhmc_ctx* ctx, const double* A, const double* B, int32_t n, double ridge,
+                    float* xt_out, int32_t* status, void* work, void* stream);
+
 /* out [n, D] = shift [D] + E [n, D] R [D, D] (fp32): draws of a Gaussian
  * N(shift, R^T R) from standard normal rows E (the Laplace warm start's
  * draws, edward/inferences/laplace.py:17-137 fits that Gaussian). */
