@@ -99,6 +99,7 @@ constexpr int kChainPad = cmax(cmax(Cfg1::BM, CfgG2::BM), cmax(CfgP2::BM, 128));
 constexpr int kRowPad = cmax(cmax(Cfg1::BN, CfgP2::BN), 128);
 static_assert(kChainPad % Cfg1::BM == 0 && kChainPad % CfgG2::BM == 0 &&
               kChainPad % CfgP2::BM == 0 && kChainPad % 128 == 0, "chain padding");
+static_assert(Cfg1::kWN == 2 && Cfg1::kWavesN == 2 && Cfg1::BN == kLLTile, "order of the log-likelihood sums");
 static_assert(kRowPad % Cfg1::BN == 0 && kRowPad % CfgP2::BN == 0, "row padding");
 constexpr int kChainThreads = 256;
 
@@ -1214,6 +1215,7 @@ static int rows_eval(edhmc_ctx* ctx, bool ll, hipStream_t st, const HierRows* hr
   RowsArgs a = {};
   a.Xp = (const float*)ctx->Xp.p;
   a.yp = (const float*)ctx->yp.p;
+  a.y = (const float*)ctx->y.p;
   a.W = (const float*)ctx->z_lp.p;
   a.N = ctx->N;
   a.N_pad = ctx->N_pad;
@@ -1226,6 +1228,7 @@ static int rows_eval(edhmc_ctx* ctx, bool ll, hipStream_t st, const HierRows* hr
   a.g_ld = ctx->g_ld;
   a.llpart = (double*)ctx->llpart.p;
   a.ll_ld = ctx->C_pad;
+  a.eta = (float*)ctx->Rt.p;
   if (hr) {
     a.goff = hr->goff;
     a.goff_ld = hr->goff_ld;
@@ -1242,7 +1245,7 @@ static int rows_eval(edhmc_ctx* ctx, bool ll, hipStream_t st, const HierRows* hr
     ProfScope ps(ctx, PK_GEMM_GRAD, st);
     EDHMC_TRY(rows_launch(ctx, a, ll, st));
   }
-  return ll ? ll_reduce(ctx, a.splits, st) : EDHMC_OK;
+  return ll ? ll_reduce(ctx, (int)(ctx->N_pad / kLLTile), st) : EDHMC_OK;
 }
 
 static int grad_eval(edhmc_ctx* ctx, bool split, bool ll, hipStream_t st) {
@@ -2043,11 +2046,6 @@ static int ensure_chains(edhmc_ctx* ctx, int C, hipStream_t st) {
                            (float*)ctx->Xs.p, st));
     }
   } else {
-    // residuals: none after a one-pass gradient but the hierarchical model's;
-    // rows up to a whole W-stationary tile, whose residual epilogue stores the
-    // last tile's rows past N_pad (zeros) without a bounds test
-    if (rows_ok(ctx) && !ctx->hier) ctx->Rt.release();
-    else EDHMC_TRY(dev_alloc(ctx, ctx->Rt, (size_t)C_pad * round_up(ctx->N_pad, kWsTile) * eb, false));
     // split-K for GEMM2: aim for >= 2048 workgroups, >= 8 stages per split.
     const int bn2 = (ctx->D_pad % Cfg1::BN == 0) ? Cfg1::BN : Cfg2S::BN;
     const int tiles2 = (C_pad / 128) * (ctx->D_pad / bn2);
@@ -2057,7 +2055,14 @@ static int ensure_chains(edhmc_ctx* ctx, int C, hipStream_t st) {
     if (ks >= 8) ks = ks / 8 * 8;
     ctx->ksplit = ks;
     ctx->g_ld = C_pad;
-    ctx->n_tiles1 = std::max(ctx->n_tiles1, ks);   // one-pass gradient: partials per range
+    // residuals, or after a one-pass gradient (but the hierarchical model's)
+    // eta of the rows whose log-likelihood is summed in a kernel of its own;
+    // rows up to a whole W-stationary tile, whose residual epilogue stores the
+    // last tile's rows past N_pad (zeros) without a bounds test
+    const size_t rt = rows_ok(ctx) && !ctx->hier
+                          ? (size_t)rows_eta(C, ks, ctx->N_pad) * 4
+                          : (size_t)C_pad * round_up(ctx->N_pad, kWsTile) * eb;
+    EDHMC_TRY(dev_alloc(ctx, ctx->Rt, rt, false));
   }
   EDHMC_TRY(dev_alloc(ctx, ctx->Gpart, (size_t)ctx->ksplit * ctx->g_ld * ctx->D_pad * 4, false));
   EDHMC_TRY(dev_alloc(ctx, ctx->llpart, (size_t)C_pad * ctx->n_tiles1 * 8, false));

@@ -49,6 +49,7 @@ namespace edhmc {
 struct RowsArgs {
   const float* Xp;         // [N_pad][DP] row-major, columns in pi order
   const float* yp;         // [N_pad], rows of every 16-row block in pi order
+  const float* y;          // [N_pad] in order
   const float* W;          // positions [>= C][DP]
   int64_t N, N_pad;
   int64_t rows_per_split;  // multiple of 16
@@ -56,8 +57,13 @@ struct RowsArgs {
   LikParams lp;
   float* Gpart;            // [splits][g_ld][DP]
   int64_t g_ld;
-  double* llpart;          // [splits][ll_ld]
+  // log-likelihood: FP64 sums over 128 rows llpart [N_pad / 128][ll_ld], and
+  // eta [C][128] of the 128-row tiles that rows_ll_kernel sums: in
+  // grad_rows_kernel all (eta + tile * C * 128), in grad_wide_kernel those that
+  // lie in two row ranges (eta + range where the tile begins * C * 128)
+  double* llpart;
   int64_t ll_ld;
+  float* eta;
   // hierarchical model: the group intercept goff[c * goff_ld + g] of each
   // row's group g (gidxp in pi order) is added to eta, and the residuals are
   // kept in Rt [N_pad / 16][ldr][16]
@@ -82,6 +88,15 @@ __host__ __device__ inline int pi16_inv(int k) {
   return 4 * (((k >> 2) & 1) | ((k & 1) << 1)) + (((k >> 1) & 1) | ((k >> 3) << 1));
 }
 
+// The log-likelihood sums its FP64 terms as EpiGLM does (a log ratio of a few
+// nats is the difference of two sums of up to a million: it shows the order
+// of the sum): the rows of every 64 by a tree over the bits of their index,
+// 5 4 3 2 1 0, then the two halves of a 128-row tile.  Summed in the order of
+// the walk instead, an evaluation with it was 20 us faster at 50 chains on
+// 100,003 x 101 and 80 at 1024 on 100,000 x 256, and log ratios of 0.05 at a
+// log joint of a million were off by 1e-9 of themselves.
+constexpr int kLLTile = 128;
+
 // 16 bytes per lane from rsrc + off to LDS at dst + 16 lane.
 __device__ inline void load_to_lds(__amdgpu_buffer_rsrc_t rsrc, float* dst, int off) {
   typedef __attribute__((address_space(3))) void lds_void;
@@ -95,6 +110,15 @@ __device__ inline void swap_halves(float& a, float& b) {
                                                   __builtin_bit_cast(uint32_t, b), false, false);
   a = __builtin_bit_cast(float, (uint32_t)r[0]);
   b = __builtin_bit_cast(float, (uint32_t)r[1]);
+}
+
+// Rows 4 h .. 4 h + 3 of a 16-row block, from the lane quarters that hold them
+// (element v of quarter h being row pi(4 h + v)).
+__device__ inline f32x4_t rows_in_order(const f32x4_t& r) {
+  float q0 = r[0], q1 = r[2], q2 = r[1], q3 = r[3];
+  swap_halves(q0, q1);
+  swap_halves(q2, q3);
+  return f32x4_t{q0, q1, q2, q3};
 }
 
 // Reads through the scalar unit (p and i uniform over the wave; nothing in the
@@ -158,7 +182,6 @@ grad_rows_kernel(RowsArgs a) {
   // distinct arrays: a direct load into one does not make reads of another wait
   __shared__ __align__(16) float x0[TR * DP], x1[TR * DP], x2[TR * DP];
   __shared__ __align__(16) float fr[2 * FR];   // fragment (b, cw) of a tile: lane * 4 + v
-  __shared__ double lsum[LL ? RW * CT : 1];
 
   int tile, split;
   if (a.splits % 8 == 0) {
@@ -191,7 +214,6 @@ grad_rows_kernel(RowsArgs a) {
   for (int i = 0; i < CW; ++i)
 #pragma unroll
     for (int k = 0; k < NC; ++k) g[i][k] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-  double lls = 0.0;
 
   // tile t into an X buffer: load i of this wave fills chunks 64 (LOADS wave +
   // i) + lane (rows past the padding: the last row, their residuals are
@@ -277,15 +299,13 @@ grad_rows_kernel(RowsArgs a) {
       for (int v = 0; v < 4; ++v) {
         const bool ok = 16 * blk + pi16(4 * h + v) < left;
         const float eta = HIER ? e[b][v] + oc[b][v] : e[b][v];
-        float dll;
-        if (LL) {
-          double ll;
-          glm_both(lp, eta, yc[b][v], dll, ll);
-          lls += ok ? ll : 0.0;
-        } else {
-          dll = glm_dll(lp, eta, yc[b][v]);
-        }
-        r[v] = ok ? dll : 0.0f;
+        r[v] = ok ? glm_dll(lp, eta, yc[b][v]) : 0.0f;
+      }
+      if (LL && 16 * blk < left) {   // not a block of the next range
+        const int64_t nb = n0 + (int64_t)t * TR + 16 * blk;
+        const f32x4_t o = rows_in_order(e[b]);
+        if (c < a.C)
+          *(f32x4_t*)(a.eta + ((nb / kLLTile) * a.C + c) * kLLTile + nb % kLLTile + 4 * h) = o;
       }
       *(f32x4_t*)(fb + (blk * CW + cw) * 256 + 4 * lane) = r;
     }
@@ -382,18 +402,6 @@ grad_rows_kernel(RowsArgs a) {
         if (cg < a.C) row[(p & ~15) + pi16(p & 15)] = g[i][k][v];
       }
     }
-  if (LL) {
-    lls += __shfl_xor(lls, 16, 64);
-    lls += __shfl_xor(lls, 32, 64);
-    if (lane < 16) lsum[rw * CT + 16 * cw + lane] = lls;
-    __syncthreads();
-    if (tid < CT) {
-      double s = 0.0;
-#pragma unroll
-      for (int w = 0; w < RW; ++w) s += lsum[w * CT + tid];
-      a.llpart[(int64_t)split * a.ll_ld + tile * CT + tid] = s;
-    }
-  }
 }
 
 // The same gradient for many chains: every wave owns 16 chains with all
@@ -448,7 +456,7 @@ grad_wide_kernel(RowsArgs a) {
   f32x4_t g[Q];
 #pragma unroll
   for (int k = 0; k < Q; ++k) g[k] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-  double lls = 0.0;
+  double la[4] = {}, lb[4] = {}, first = 0.0;   // even and odd blocks of 64 rows; 64 rows' sum
 
   int loff[LOADS];
 #pragma unroll
@@ -554,19 +562,56 @@ grad_wide_kernel(RowsArgs a) {
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  // residual of element v of block b of tile t, in place
-  auto residual = [&](int t, f32x4_t (&e)[RB], int b, int v) {
-    const bool ok = t * TR + 16 * b + pi16(4 * h + v) < rows;
-    const float eta = HIER ? e[b][v] + oc[b][v] : e[b][v];
-    float dll;
-    if (LL) {
-      double ll;
-      glm_both(lp, eta, yc[b][v], dll, ll);
-      lls += ok ? ll : 0.0;
+  // terms x of a block of rows from nb on (zeros past N) into their 128-row
+  // tile's sum
+  auto ll_block = [&](int64_t nb, const double (&x)[4]) {
+    const int p = (int)(nb >> 4) & 7;
+    if (p & 1) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) lb[v] += x[v];
     } else {
-      dll = glm_dll(lp, eta, yc[b][v]);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) la[v] += x[v];
     }
-    e[b][v] = ok ? dll : 0.0f;
+    const bool last = nb + 16 >= n_end;
+    if ((p & 3) != 3 && !last) return;
+    double s0 = (la[0] + lb[0]) + (la[2] + lb[2]), s1 = (la[1] + lb[1]) + (la[3] + lb[3]);
+    s0 += __shfl_xor(s0, 16, 64);
+    s1 += __shfl_xor(s1, 16, 64);
+    double s = s0 + s1;
+    s += __shfl_xor(s, 32, 64);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) la[v] = lb[v] = 0.0;
+    first = p < 4 ? s : first + s;
+    if ((p == 7 || last) && lane < 16 && c < a.C) a.llpart[nb / kLLTile * a.ll_ld + c] = first;
+  };
+  // residuals of block b of tile t, in place
+  auto residual = [&](int t, f32x4_t (&e)[RB], int b) {
+    const int64_t nb = n0 + (int64_t)t * TR + 16 * b;
+    bool here = false;    // its 128-row tile lies within this range
+    if (LL && nb < n_end) {
+      const int64_t tb = nb / kLLTile * kLLTile;
+      here = tb >= n0 && tb + kLLTile <= n0 + a.rows_per_split;
+      if (!here && c < a.C)
+        *(f32x4_t*)(a.eta + (tb / a.rows_per_split * a.C + c) * kLLTile + nb % kLLTile + 4 * h) =
+            rows_in_order(e[b]);
+    }
+    double x[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const bool ok = t * TR + 16 * b + pi16(4 * h + v) < rows;
+      const float eta = HIER ? e[b][v] + oc[b][v] : e[b][v];
+      float dll;
+      if (LL) {
+        double ll;
+        glm_both(lp, eta, yc[b][v], dll, ll);
+        x[v] = ok ? ll : 0.0;
+      } else {
+        dll = glm_dll(lp, eta, yc[b][v]);
+      }
+      e[b][v] = ok ? dll : 0.0f;
+    }
+    if (LL && here) ll_block(nb, x);
   };
   // GEMM2 of a tile
   auto gemm2 = [&](const float* xb, const f32x4_t (&r)[RB]) {
@@ -605,11 +650,7 @@ grad_wide_kernel(RowsArgs a) {
     for (int b = 0; b < RB; ++b) {
       const int64_t nb = n0 + (int64_t)t * TR + 16 * b;   // first row of the block
       if (nb >= n_end) break;
-      // rows 4 h .. 4 h + 3 of the block, from the quarters that hold them
-      float q0 = r[b][0], q1 = r[b][2], q2 = r[b][1], q3 = r[b][3];
-      swap_halves(q0, q1);
-      swap_halves(q2, q3);
-      const f32x4_t q = {q0, q1, q2, q3};
+      const f32x4_t q = rows_in_order(r[b]);
       bool keep = !inside;
       const int64_t be = min(nb + 16, n_end);
       if (gend > be) {   // the block lies within one group that goes on
@@ -665,8 +706,7 @@ grad_wide_kernel(RowsArgs a) {
     rows_of(t_ + 1);                                                     \
     if constexpr (HIER) offsets_of();                                    \
     gemm1(XT, e);                                                        \
-    _Pragma("unroll") for (int i = 0; i < 4 * RB; ++i)                   \
-      residual(t_, e, i / 4, i % 4);                                     \
+    _Pragma("unroll") for (int b = 0; b < RB; ++b) residual(t_, e, b);   \
     gemm2(XT, e);                                                        \
     if constexpr (HIER) segments(t_, e);                                 \
     rotate(t_ + 1);                                                      \
@@ -697,10 +737,50 @@ grad_wide_kernel(RowsArgs a) {
     const f32x4_t v = *(const f32x4_t*)(own + r * DP + 4 * (u ^ r));
     if (c0 + r < a.C) *(f32x4_t*)(a.Gpart + ((int64_t)split * a.g_ld + c0 + r) * DP + 4 * u) = v;
   }
-  if (LL) {
-    lls += __shfl_xor(lls, 16, 64);
-    lls += __shfl_xor(lls, 32, 64);
-    if (lane < 16) a.llpart[(int64_t)split * a.ll_ld + c] = lls;
+}
+
+// The FP64 sums of the tiles whose eta was kept, eight chains per workgroup:
+// all tiles, or (wide) one per end of a row range and the tile of padding that
+// may come last.
+template <bool BERN>
+__global__ void __launch_bounds__(256)
+rows_ll_kernel(RowsArgs a, bool wide) {
+  const int l = threadIdx.x & 31, c = blockIdx.x * 8 + (threadIdx.x >> 5);
+  if (c >= a.C) return;
+  LikParams lp = a.lp;
+  lp.lik = BERN ? LIK_BERNOULLI : LIK_NORMAL;
+  const int64_t tiles = a.N_pad / kLLTile, slots = wide ? a.splits + 1 : tiles;
+  for (int64_t slot = blockIdx.y; slot < slots; slot += gridDim.y) {
+    int64_t tile = slot;
+    if (wide && slot < a.splits) {
+      const int64_t e = (slot + 1) * a.rows_per_split;   // in two ranges, of which this is the first
+      tile = e / kLLTile;
+      if (e % kLLTile == 0 || tile >= tiles || tile * kLLTile / a.rows_per_split != slot) continue;
+    } else if (wide) {
+      tile = tiles - 1;
+      if (tile * kLLTile < a.N) continue;
+    }
+    const float* eta = a.eta + (slot * a.C + c) * kLLTile;
+    double s = 0.0;
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      double q = 0.0;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int r = 64 * half + 32 * j + l;
+        const int64_t n = tile * kLLTile + r;
+        if (n < a.N) {
+          float dll;
+          double ll;
+          glm_both(lp, eta[r], a.y[n], dll, ll);
+          q += ll;
+        }
+      }
+#pragma unroll
+      for (int off = 16; off > 0; off >>= 1) q += __shfl_xor(q, off, 64);
+      s += q;
+    }
+    if (l == 0) a.llpart[tile * a.ll_ld + c] = s;
   }
 }
 
@@ -708,6 +788,8 @@ grad_wide_kernel(RowsArgs a) {
 bool rows_ok(const edhmc_ctx* ctx);
 // Whether a call of C chains over this many row ranges takes grad_wide_kernel.
 bool rows_wide(int C, int splits);
+// Floats that RowsArgs.eta holds.
+int64_t rows_eta(int C, int splits, int64_t N_pad);
 // Fills in the chain tiles (C, splits set) and launches.
 int rows_launch(edhmc_ctx* ctx, RowsArgs a, bool ll, hipStream_t st);
 // out[16 b + p] = in[16 b + pi(p)] for n values (a multiple of 16), 4 bytes each.

@@ -67,6 +67,10 @@ static void launch_dp(const RowsArgs& a, bool ll, hipStream_t st) {
   launch_cw<DP, 2>(a, ll, st);
 }
 
+int64_t rows_eta(int C, int splits, int64_t N_pad) {
+  return rows_wide(C, splits) ? (int64_t)splits * C * kLLTile : N_pad * C;
+}
+
 int rows_launch(edhmc_ctx* ctx, RowsArgs a, bool ll, hipStream_t st) {
   if ((a.rows_per_split + 256) * ctx->D_pad * 4 > 0x7fffffffLL)
     return set_err(ctx, EDHMC_EUNSUPPORTED, "one-pass gradient: row range too long");
@@ -77,7 +81,14 @@ int rows_launch(edhmc_ctx* ctx, RowsArgs a, bool ll, hipStream_t st) {
     case 256: launch_dp<256>(a, ll, st); break;
     default: return set_err(ctx, EDHMC_EUNSUPPORTED, "one-pass gradient: D_pad %d", ctx->D_pad);
   }
-  return check_launch(ctx, "grad_rows");
+  EDHMC_TRY(check_launch(ctx, "grad_rows"));
+  if (!ll) return EDHMC_OK;
+  const bool wide = rows_wide(a.C, a.splits);
+  const int64_t slots = wide ? a.splits + 1 : a.N_pad / kLLTile;
+  const dim3 grid((a.C + 7) / 8, (unsigned)std::min<int64_t>(slots, 4096));
+  if (a.lp.lik == LIK_BERNOULLI) hipLaunchKernelGGL((rows_ll_kernel<true>), grid, dim3(256), 0, st, a, wide);
+  else hipLaunchKernelGGL((rows_ll_kernel<false>), grid, dim3(256), 0, st, a, wide);
+  return check_launch(ctx, "rows_ll");
 }
 
 __global__ void __launch_bounds__(256)
