@@ -79,6 +79,7 @@ SIGNATURES = {
     'edhmc_draw_momenta': (ctypes.c_int, [_c_p, _i32, _i32, _u64, _u64, _c_p, _c_p]),
     'edhmc_draw_uniforms': (ctypes.c_int, [_c_p, _i32, _u64, _u64, _c_p, _c_p]),
     'edhmc_autocov': (ctypes.c_int, [_c_p, _c_p, _i64, _i32, _i32, _i32, _c_p, _c_p, _c_p]),
+    'edhmc_ess': (ctypes.c_int, [_c_p, _c_p, _i64, _i32, _i32, _i32, _c_p, _c_p]),
     'edhmc_autocov_lags': (ctypes.c_int, [_c_p, _c_p, _i64, _i32, _i32, _i32, _i32, _c_p, _c_p,
                                           _c_p]),
     'edhmc_sur_create': (ctypes.c_int, [_c_p, _i32, _i32, _i32]),

@@ -2208,7 +2208,7 @@ edhmc_ctx::~edhmc_ctx() {
   DevBuf* bufs[] = {&Xr, &Xc, &Xf, &Xs, &Xp, &yp, &y, &ploc, &pscale, &z, &r, &g, &z0, &g0, &z_lp, &logp, &K0,
                     &flag, &ndiv, &ratio, &Rt, &Gpart, &llpart, &ll, &mom_mean, &mom_m2, &tmp_count,
                     &stats_part, &pred_col, &ll_split, &pkind, &plnorm,
-                    &newton, &acov_part, &acov_mean};
+                    &newton, &acov_part, &acov_mean, &acov_rows, &acov, &ess_spread};
   for (DevBuf* b : bufs) b->release();
 }
 

@@ -13,102 +13,105 @@
 
 using namespace edhmc;
 
+namespace edhmc {
+bool autocov_fft_ok(int64_t T, int n_lags);
+int autocov_fft(edhmc_ctx* ctx, const float* s, int64_t T, int C, int D, int n_lags, double* mean,
+                double* acov, hipStream_t st);
+int ess_launch(edhmc_ctx* ctx, const double* acov, const double* mean, int64_t T, int C, int D,
+               bool between, double* ess, hipStream_t st);
+}  // namespace edhmc
+
 namespace {
 
 // ---------------------------------------------------------------------------
-// Column moments of x [T, K] over rows t0 .. T-1: two-pass mean and
-// population variance (var == nullptr: the mean alone).
+// Column moments of x [T, K] over rows t0 .. T-1: mean and population variance
+// (var == nullptr: the mean alone).
 //
-// A workgroup of 1024 threads takes CW columns and deals the rows round-robin
-// to 1024 / CW groups of threads.  With R > 0 (rows <= R 1024 / CW) a thread
-// keeps its rows in registers, so x is read once and 32 loads are in flight
-// per thread; with R = 0 the second pass reads x again.  Bound by the read of
-// x: T = 1000, K = 262,144 (1.05 GB) in 616 us against 906 us for a thread
-// per column in two dependent passes.  CW = 64 columns, or fewer for a store
-// of fewer columns, so that one chain's store of thousands of rows still
-// fills a workgroup.
+// A workgroup of NT threads takes CW adjacent columns and deals the rows
+// round-robin to NT / CW groups of threads.  A thread takes kMomRows rows at
+// a time, the next ones loading meanwhile, and merges their sum and squared
+// deviations from their own mean into its running ones (Chan, Golub, LeVeque
+// 1979), so x is read once whatever T is, 1 KB of a row at a time in a wide
+// store.  Bound by the read of x; T = 1000, K = 262,144 (1.05 GB): 210
+// us, 5.0 TB/s (64 columns at a time, the rows in registers: 616).
 // ---------------------------------------------------------------------------
-constexpr int kMomThreads = 1024;
+constexpr int kMomRows = 16;
 
-// Sum over the row groups (a power of two), every thread of a column.
-__device__ inline double group_sum(double v, double* sm, int tid, int cw) {
-  __syncthreads();
-  sm[tid] = v;
-  __syncthreads();
-  for (int w = kMomThreads / 2; w >= cw; w >>= 1) {
-    if (tid < w) sm[tid] += sm[tid + w];
-    __syncthreads();
-  }
-  return sm[tid & (cw - 1)];
+struct Moments {
+  double n, sum, dev;   // rows, their sum, squared deviations from their mean
+};
+
+__device__ inline Moments merge(const Moments& a, const Moments& b) {
+  if (b.n == 0.0) return a;
+  if (a.n == 0.0) return b;
+  const double n = a.n + b.n, d = b.sum / b.n - a.sum / a.n;
+  return {n, a.sum + b.sum, a.dev + b.dev + d * d * (a.n * b.n / n)};
 }
 
-template <typename P, int R>
-__global__ void __launch_bounds__(kMomThreads)
+template <typename P, int NT>
+__global__ void __launch_bounds__(NT)
 moments_kernel(const P* __restrict__ x, int64_t T, int64_t K, int64_t t0, int cw,
                double* __restrict__ mean, double* __restrict__ var) {
-  __shared__ double sm[kMomThreads];
-  const int tid = threadIdx.x, groups = kMomThreads / cw;
+  __shared__ Moments sm[NT];
+  const int tid = threadIdx.x, groups = NT / cw;
   const int64_t k = (int64_t)blockIdx.x * cw + (tid & (cw - 1));
   const int g = tid / cw;
-  const bool kv = k < K;
   const int64_t n = T - t0;
-  const P* p = x + (t0 + g) * K + (kv ? k : 0);
+  const int64_t mine = g < n ? (n - g + groups - 1) / groups : 0;   // rows g, g + groups, ...
+  const P* p = x + (t0 + g) * K + min(k, K - 1);
   const int64_t step = (int64_t)groups * K;
-  P v[R > 0 ? R : 1];
-  double s = 0.0;
-  if constexpr (R > 0) {
+  P v[kMomRows];
+  auto load = [&](int64_t i0) {
 #pragma unroll
-    for (int i = 0; i < R; ++i) v[i] = g + (int64_t)i * groups < n ? p[i * step] : (P)0;
+    for (int i = 0; i < kMomRows; ++i) v[i] = i0 + i < mine ? p[(i0 + i) * step] : (P)0;
+  };
+  Moments a = {0.0, 0.0, 0.0};
+  load(0);
+  for (int64_t i0 = 0; i0 < mine; i0 += kMomRows) {
+    P w[kMomRows];
 #pragma unroll
-    for (int i = 0; i < R; ++i) s += (double)v[i];
-  } else {
-    int64_t i = g;
-    const P* q = p;
-#pragma unroll 8
-    for (; i < n; i += groups, q += step) s += (double)*q;
-  }
-  const double m = group_sum(s, sm, tid, cw) / (double)n;
-  if (kv && g == 0) mean[k] = m;
-  if (!var) return;   // uniform across the grid
-  double q2 = 0.0;
-  if constexpr (R > 0) {
+    for (int i = 0; i < kMomRows; ++i) w[i] = v[i];
+    if (i0 + kMomRows < mine) load(i0 + kMomRows);
+    const int cnt = (int)min((int64_t)kMomRows, mine - i0);
+    Moments b = {(double)cnt, 0.0, 0.0};
 #pragma unroll
-    for (int i = 0; i < R; ++i) {
-      const double d = (double)v[i] - m;
-      q2 += g + (int64_t)i * groups < n ? d * d : 0.0;
+    for (int i = 0; i < kMomRows; ++i) b.sum += (double)w[i];   // zeros from cnt on
+    const double m = b.sum / b.n;
+#pragma unroll
+    for (int i = 0; i < kMomRows; ++i) {
+      const double d = (double)w[i] - m;
+      b.dev += i < cnt ? d * d : 0.0;
     }
-  } else {
-    int64_t i = g;
-    const P* q = p;
-#pragma unroll 8
-    for (; i < n; i += groups, q += step) {
-      const double d = (double)*q - m;
-      q2 += d * d;
-    }
+    a = merge(a, b);
   }
-  q2 = group_sum(q2, sm, tid, cw);
-  if (kv && g == 0) var[k] = q2 / (double)n;
+  sm[tid] = a;
+  __syncthreads();
+  for (int w = NT / 2; w >= cw; w >>= 1) {
+    if (tid < w) sm[tid] = merge(sm[tid], sm[tid + w]);
+    __syncthreads();
+  }
+  if (g != 0 || k >= K) return;
+  a = sm[tid];
+  mean[k] = a.sum / a.n;
+  if (var) var[k] = a.dev / a.n;
 }
 
 template <typename P>
 int launch_moments(edhmc_ctx* ctx, const P* x, int64_t T, int64_t K, int64_t t0, double* mean,
                    double* var, hipStream_t st) {
-  // columns per workgroup: 64, halved down to 16 while that lets 32 rows per
-  // thread hold them all (up to 2048 rows), fewer for a narrow store
+  // columns per workgroup: 256 where that leaves a thousand workgroups, down
+  // to 64, fewer for a narrow store; 1024 threads (rows in more groups) where
+  // there are few workgroups
   int cw = 4;
   while (cw < 64 && cw < K) cw *= 2;
-  const int64_t n = T - t0;
-  auto per = [&](int w) { return (n + kMomThreads / w - 1) / (kMomThreads / w); };
-  while (cw > 16 && per(cw) > 32 && per(16) <= 32) cw /= 2;
+  while (cw >= 64 && cw < 256 && K / (2 * cw) >= 1024) cw *= 2;
   const int64_t blocks = (K + cw - 1) / cw;
   if (blocks > 2147483647LL) return set_err(ctx, EDHMC_EUNSUPPORTED, "too many columns");
-  const dim3 grid((unsigned)blocks), block(kMomThreads);
-  if (per(cw) <= 8)
-    hipLaunchKernelGGL((moments_kernel<P, 8>), grid, block, 0, st, x, T, K, t0, cw, mean, var);
-  else if (per(cw) <= 32)
-    hipLaunchKernelGGL((moments_kernel<P, 32>), grid, block, 0, st, x, T, K, t0, cw, mean, var);
+  const dim3 grid((unsigned)blocks);
+  if (blocks >= 1024)
+    hipLaunchKernelGGL((moments_kernel<P, 256>), grid, dim3(256), 0, st, x, T, K, t0, cw, mean, var);
   else
-    hipLaunchKernelGGL((moments_kernel<P, 0>), grid, block, 0, st, x, T, K, t0, cw, mean, var);
+    hipLaunchKernelGGL((moments_kernel<P, 1024>), grid, dim3(1024), 0, st, x, T, K, t0, cw, mean, var);
   return check_launch(ctx, "moments");
 }
 
@@ -124,10 +127,11 @@ int launch_moments(edhmc_ctx* ctx, const P* x, int64_t T, int64_t K, int64_t t0,
 // register arrays) and issues 256 FP64 FMAs; the four waves of a workgroup
 // take adjacent lag blocks of the same columns, and the workgroups of one
 // column strip and chain group run on one XCD, so the store is read from its
-// L2.  Bound by the FP64 FMAs (n_lags (T - lag) C D of them).  T = 1000,
-// C = 1024, D = 256, the five windows of an effective sample size that needs
-// all 1000 lags: 14.8 ms, against 105 ms for a thread per series with one
-// atomic per series and lag and every widening from lag 0.
+// L2.  Bound by the FP64 FMAs (n_lags (T - lag) C D of them) and the wait
+// for the loads.  T = 1000, C = 1024, D = 256, all 1000 lags in five windows:
+// 14.8 ms, against 105 ms for a thread per series with one atomic per series
+// and lag.  It takes windows that do not begin at lag 0, at most 32 lags, and
+// more than 2048 draws (acov_fft.hip the others).
 // ---------------------------------------------------------------------------
 constexpr int kAcLags = 32, kAcStep = 8, kAcWaves = 4;
 constexpr int kAcWin = kAcLags / kAcStep + 1;   // window of kAcWin kAcStep values
@@ -280,7 +284,22 @@ int autocov_lags(edhmc_ctx* ctx, const float* s, int64_t T, int C, int D, int la
   return check_launch(ctx, "autocov_sum");
 }
 
+// Lags 0 .. n_lags - 1 and the chain means they take.
+int autocov_from_zero(edhmc_ctx* ctx, const float* s, int64_t T, int C, int D, int n_lags,
+                      double* mean, double* acov, hipStream_t st) {
+  if (autocov_fft_ok(T, n_lags)) return autocov_fft(ctx, s, T, C, D, n_lags, mean, acov, st);
+  EDHMC_TRY(launch_moments<float>(ctx, s, T, (int64_t)C * D, 0, mean, nullptr, st));
+  return autocov_lags(ctx, s, T, C, D, 0, n_lags, mean, acov, st);
+}
+
 }  // namespace
+
+namespace edhmc {
+int moments_f64(edhmc_ctx* ctx, const double* x, int64_t T, int64_t K, double* mean, double* var,
+                hipStream_t st) {
+  return launch_moments<double>(ctx, x, T, K, 0, mean, var, st);
+}
+}  // namespace edhmc
 
 extern "C" {
 
@@ -313,8 +332,22 @@ int edhmc_autocov(edhmc_ctx* ctx, const float* s, int64_t T, int32_t C, int32_t 
     EDHMC_TRY(dev_reserve(ctx, ctx->acov_mean, (size_t)K * 8));
     mean = (double*)ctx->acov_mean.p;
   }
-  EDHMC_TRY(launch_moments<float>(ctx, s, T, K, 0, mean, nullptr, st));
-  return autocov_lags(ctx, s, T, C, D, 0, max_lag + 1, mean, acov_out, st);
+  return autocov_from_zero(ctx, s, T, C, D, max_lag + 1, mean, acov_out, st);
+}
+
+int edhmc_ess(edhmc_ctx* ctx, const float* s, int64_t T, int32_t C, int32_t D, int32_t between,
+              double* ess_out, void* stream) {
+  if (!ctx) return EDHMC_EINVAL;
+  DeviceGuard dg(ctx->device);
+  hipStream_t st = (hipStream_t)stream;
+  if (!s || !ess_out || T < 4 || T > 2147483647LL || C <= 0 || D <= 0)
+    return set_err(ctx, EDHMC_EINVAL, "bad arguments");
+  EDHMC_TRY(dev_reserve(ctx, ctx->acov_mean, (size_t)C * D * 8));
+  EDHMC_TRY(dev_reserve(ctx, ctx->acov, (size_t)T * D * 8));
+  double* mean = (double*)ctx->acov_mean.p;
+  double* acov = (double*)ctx->acov.p;
+  EDHMC_TRY(autocov_from_zero(ctx, s, T, C, D, (int)T, mean, acov, st));
+  return ess_launch(ctx, acov, mean, T, C, D, between != 0, ess_out, st);
 }
 
 int edhmc_autocov_lags(edhmc_ctx* ctx, const float* s, int64_t T, int32_t C, int32_t D,

@@ -19,6 +19,9 @@ import torch
 from edward_amd import _lib as L
 
 
+_ALL_LAGS = 2048   # draws up to which edhmc_autocov sums every lag at once
+
+
 def autocov(engine, samples, max_lag):
   """Sum over chains of each chain's biased autocovariance at lags
   0..max_lag, [max_lag+1, D] fp64, plus chain means [C, D]."""
@@ -79,13 +82,19 @@ def _ess_from_spread(acov_sum, spread, M, n):
 
 
 def ess(engine, samples, max_lag=64, between=True):
-  """Per-coordinate ESS of samples [T, C, D] (device, fp32); the lag window
-  doubles until every coordinate's Geyer sequence is truncated (each lag is
-  summed once)."""
+  """Per-coordinate ESS of samples [T, C, D] (device, fp32).  Up to 2048
+  draws all lags come from one transform per pair of chains and are summed
+  on the device (``edhmc_ess``); beyond, the lag window doubles until every
+  coordinate's Geyer sequence is truncated (each lag is summed once)."""
   T, M, D = (int(v) for v in samples.shape)
   if T < 4:
     return np.full(D, np.nan)   # too few draws to estimate
   s = samples.contiguous()
+  if T <= _ALL_LAGS:
+    out = torch.empty(D, dtype=torch.float64, device=s.device)
+    engine.check(engine.lib.edhmc_ess(engine.h, L.ptr(s), T, M, D, int(bool(between)), L.ptr(out),
+                                      engine.stream))
+    return out.cpu().numpy()
   lag = min(max_lag, T - 1)
   acov, cmean = autocov(engine, s, lag)
   acov = acov.cpu().numpy()

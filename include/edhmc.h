@@ -330,6 +330,12 @@ int edhmc_draw_uniforms(edhmc_ctx* ctx, int32_t C, uint64_t seed, uint64_t count
 int edhmc_autocov(edhmc_ctx* ctx, const float* s, int64_t T, int32_t C, int32_t D,
                   int32_t max_lag, double* acov_out, double* chain_mean_out,
                   void* stream);
+/* Effective sample size of each coordinate over the chains of s [T, C, D]
+ * fp32 (T >= 4), ess_out [D] fp64: all T lags, Geyer's initial positive and
+ * monotone sequence, with between != 0 and C > 1 the variance of the chain
+ * means beside that within the chains; 0 where nothing moved. */
+int edhmc_ess(edhmc_ctx* ctx, const float* s, int64_t T, int32_t C, int32_t D, int32_t between,
+              double* ess_out, void* stream);
 /* The same autocovariances at lags lag0 .. lag0 + n_lags - 1 only
  * (lag0 + n_lags <= T), acov_out [n_lags, D] fp64, from the chain means
  * [C, D] fp64 that edhmc_autocov wrote for the same store: a window that
