@@ -24,6 +24,7 @@
 #include "gemm2_dma.h"
 #include "few_chains.h"
 #include "grad_rows.h"
+#include "predict.h"
 #include "philox.h"
 #include "transform.h"
 
@@ -368,15 +369,16 @@ replicate_kernel(float* __restrict__ rep, int S, int64_t N, int lik, float scale
   }
 }
 
-// mean_out[n] = (sum over M tiles of colsum[tm][n]) / S
+// mean_out[n] = (sum over M tiles of colsum[tm][n]) / S, in FP64: with 16
+// partial sums of 32 draws an fp32 sum would round more than one of 4 of 128.
 __global__ void __launch_bounds__(256)
-colsum_reduce_kernel(const float* __restrict__ part, int m_tiles, int64_t ld, int64_t N, float inv_s,
+colsum_reduce_kernel(const float* __restrict__ part, int m_tiles, int64_t ld, int64_t N, int S,
                      float* __restrict__ out) {
   const int64_t n = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (n >= N) return;
-  float s = 0.0f;
-  for (int t = 0; t < m_tiles; ++t) s += part[(int64_t)t * ld + n];
-  out[n] = s * inv_s;
+  double s = 0.0;
+  for (int t = 0; t < m_tiles; ++t) s += (double)part[(int64_t)t * ld + n];
+  out[n] = (float)(s / (double)S);
 }
 
 // ---------------------------------------------------------------------------
@@ -2423,15 +2425,37 @@ int edhmc_predict(edhmc_ctx* ctx, const float* W, int32_t S, float* mean_out, do
       hipStreamSynchronize(st) != hipSuccess)
     return set_err(ctx, EDHMC_EHIP, "predict: copy failed");
   if (bad) return set_err(ctx, EDHMC_ENONFINITE, "draws contain %d non-finite rows", bad);
-  if (ctx->cdt == EDHMC_BF16)
+  int cols = ctx->C_pad / (ctx->cdt == EDHMC_BF16 ? CfgP2::BM : Cfg1::BM);
+  if (predict_ok(ctx) && !rep_out) {   // replicates: the general kernel stores the mean responses
+    const PredictPlan p = predict_plan(ctx, S);
+    cols = p.cols;
+    if (mean_out) EDHMC_TRY(dev_alloc(ctx, ctx->pred_col, (size_t)cols * ctx->N_pad * 4, false));
+    PredictArgs pa = {};
+    pa.Xp = (const float*)ctx->Xp.p;
+    pa.y = (const float*)ctx->y.p;
+    pa.W = (const float*)ctx->z_lp.p;
+    pa.N = ctx->N;
+    pa.N_pad = ctx->N_pad;
+    pa.D_pad = ctx->D_pad;
+    pa.S = S;
+    pa.lp = lik_params(ctx);
+    pa.llpart = (double*)ctx->llpart.p;
+    pa.ll_ld = ctx->C_pad;
+    pa.colsum = mean_out ? (float*)ctx->pred_col.p : nullptr;
+    pa.col_ld = ctx->N_pad;
+    {
+      ProfScope ps(ctx, PK_GEMM_LL, st);
+      EDHMC_TRY(predict_launch(ctx, pa, p, st));
+    }
+    EDHMC_TRY(ll_reduce(ctx, p.splits, st));
+  } else if (ctx->cdt == EDHMC_BF16)
     EDHMC_TRY((launch_predict<bf16_t, CfgP2, 2>(ctx, S, mean_out != nullptr, rep_out, seed, st)));
   else
     EDHMC_TRY((launch_predict<float, Cfg1, 1>(ctx, S, mean_out != nullptr, rep_out, seed, st)));
   if (mean_out) {
-    const int m_tiles = ctx->C_pad / (ctx->cdt == EDHMC_BF16 ? CfgP2::BM : Cfg1::BM);
     hipLaunchKernelGGL(colsum_reduce_kernel, dim3((unsigned)((ctx->N + 255) / 256)), dim3(256), 0,
-                       st, (const float*)ctx->pred_col.p, m_tiles, ctx->N_pad, ctx->N,
-                       1.0f / (float)S, mean_out);
+                       st, (const float*)ctx->pred_col.p, cols, ctx->N_pad, ctx->N, S,
+                       mean_out);
     EDHMC_TRY(check_launch(ctx, "colsum_reduce"));
   }
   if (loglik_out && hipMemcpyAsync(loglik_out, ctx->ll.p, (size_t)S * 8, hipMemcpyDeviceToDevice,
