@@ -25,6 +25,7 @@
 #include "few_chains.h"
 #include "grad_rows.h"
 #include "predict.h"
+#include "small_run.h"
 #include "philox.h"
 #include "transform.h"
 
@@ -2102,9 +2103,47 @@ static int do_set_state(edhmc_ctx* ctx, const float* W, int C, hipStream_t st) {
   return EDHMC_OK;
 }
 
-static int do_transition(edhmc_ctx* ctx, float eps, int L, const float* r0, const double* u,
-                         uint64_t seed, uint64_t counter, int32_t* accepted_out,
-                         float* sample_out, int32_t* n_accept, hipStream_t st) {
+// Transitions `counter` .. counter + T - 1 in one launch (small_run.h).
+static int do_small(edhmc_ctx* ctx, float eps, int L, const float* r0, const double* u,
+                    uint64_t seed, uint64_t counter, int T, int32_t* accepted_out,
+                    float* sample_out, int32_t* n_accept, hipStream_t st) {
+  SmallArgs a = {};
+  a.X = (const float*)ctx->Xr.p;
+  a.y = (const float*)ctx->y.p;
+  a.N = ctx->N;
+  a.D = ctx->D; a.D_pad = ctx->D_pad; a.C = ctx->C; a.L = L; a.T = T;
+  a.lp = lik_params(ctx);
+  a.lik_weight = ctx->lik_weight;
+  a.half = (float)(0.5 * (double)eps);
+  a.full = eps;
+  a.ploc = (const float*)ctx->ploc.p; a.pscale = (const float*)ctx->pscale.p;
+  a.z = (float*)ctx->z.p; a.r = (float*)ctx->r.p; a.g = (float*)ctx->g.p;
+  a.z0 = (float*)ctx->z0.p; a.g0 = (float*)ctx->g0.p; a.z_lp = (float*)ctx->z_lp.p;
+  a.logp = (double*)ctx->logp.p; a.K0 = (double*)ctx->K0.p;
+  a.r_fed = r0; a.u_fed = u;
+  a.seed = seed; a.counter = counter;
+  a.sample_out = sample_out; a.accepted_out = accepted_out; a.n_accept = n_accept;
+  a.ndiv = (int32_t*)ctx->ndiv.p;
+  a.ratio_out = (double*)ctx->ratio.p;
+  if (ctx->mom_on) {
+    a.mom_mean = (double*)ctx->mom_mean.p;
+    a.mom_m2 = (double*)ctx->mom_m2.p;
+    a.mom_n = ctx->mom_count;
+    ctx->mom_count += T;
+  }
+  ProfScope ps(ctx, PK_CHAIN, st);
+  return small_launch(ctx, a, st);
+}
+
+static int one_transition(edhmc_ctx* ctx, float eps, int L, const float* r0, const double* u,
+                          uint64_t seed, uint64_t counter, int32_t* accepted_out,
+                          float* sample_out, int32_t* n_accept, hipStream_t st);
+
+// T transitions from `counter` on, sample_out [T][C][D] (or null); fed momenta
+// and uniforms and accepted_out are for T = 1.
+static int do_transitions(edhmc_ctx* ctx, float eps, int L, const float* r0, const double* u,
+                          uint64_t seed, uint64_t counter, int64_t T, int32_t* accepted_out,
+                          float* sample_out, int32_t* n_accept, hipStream_t st) {
   if (!ctx->bound || !ctx->state_valid)
     return set_err(ctx, EDHMC_ESTATE, "no chain state: call edhmc_set_state first");
   if (L < 1) return set_err(ctx, EDHMC_EINVAL, "n_steps must be >= 1, got %d", L);
@@ -2118,6 +2157,25 @@ static int do_transition(edhmc_ctx* ctx, float eps, int L, const float* r0, cons
     ctx->g_valid = true;
   }
   surrogate_invalidate(ctx->sur);
+  const int64_t row = (int64_t)ctx->C * ctx->D;
+  if (small_ok(ctx) && L <= 65536) {
+    // launches of at most 4096 leapfrog steps or so
+    const int64_t per = std::max(1, 4096 / L);
+    for (int64_t t = 0; t < T; t += per)
+      EDHMC_TRY(do_small(ctx, eps, L, r0, u, seed, counter + (uint64_t)t,
+                         (int)std::min(per, T - t), accepted_out,
+                         sample_out ? sample_out + t * row : nullptr, n_accept, st));
+    return EDHMC_OK;
+  }
+  for (int64_t t = 0; t < T; ++t)
+    EDHMC_TRY(one_transition(ctx, eps, L, r0, u, seed, counter + (uint64_t)t, accepted_out,
+                             sample_out ? sample_out + t * row : nullptr, n_accept, st));
+  return EDHMC_OK;
+}
+
+static int one_transition(edhmc_ctx* ctx, float eps, int L, const float* r0, const double* u,
+                          uint64_t seed, uint64_t counter, int32_t* accepted_out,
+                          float* sample_out, int32_t* n_accept, hipStream_t st) {
   ChainArgs a = chain_args(ctx);
   a.half = (float)(0.5 * (double)eps);
   a.full = eps;
@@ -2469,8 +2527,8 @@ int edhmc_transition(edhmc_ctx* ctx, float eps, int32_t n_steps, const float* r0
                      int32_t* n_accept, void* stream) {
   if (!ctx) return EDHMC_EINVAL;
   DeviceGuard dg(ctx->device);
-  return do_transition(ctx, eps, n_steps, r0, u, seed, counter, accepted_out, sample_out,
-                       n_accept, (hipStream_t)stream);
+  return do_transitions(ctx, eps, n_steps, r0, u, seed, counter, 1, accepted_out, sample_out,
+                        n_accept, (hipStream_t)stream);
 }
 
 static int sg_step(edhmc_ctx* ctx, bool hamiltonian, float lr, float friction, float* v,
@@ -2719,12 +2777,10 @@ int edhmc_run(edhmc_ctx* ctx, float eps, int32_t n_steps, float* params, int64_t
   if (t0 < 0 || n_iter < 0 || t0 + n_iter > T)
     return set_err(ctx, EDHMC_EINVAL, "iterations [%lld, %lld) outside params of %lld rows",
                    (long long)t0, (long long)(t0 + n_iter), (long long)T);
-  for (int64_t t = t0; t < t0 + n_iter; ++t) {
-    EDHMC_TRY(do_transition(ctx, eps, n_steps, nullptr, nullptr, seed, counter0 + (uint64_t)t,
-                            nullptr, params + t * (int64_t)ctx->C * ctx->D, n_accept,
-                            (hipStream_t)stream));
-  }
-  return EDHMC_OK;
+  if (n_iter == 0) return EDHMC_OK;
+  return do_transitions(ctx, eps, n_steps, nullptr, nullptr, seed, counter0 + (uint64_t)t0, n_iter,
+                        nullptr, params + t0 * (int64_t)ctx->C * ctx->D, n_accept,
+                        (hipStream_t)stream);
 }
 
 int edhmc_profile_enable(edhmc_ctx* ctx, int32_t enable) {
