@@ -210,9 +210,9 @@ struct EpiPre<Epi, Cfg, std::void_t<decltype(std::declval<const Epi&>().template
   }
 };
 
+// Workgroup `id` of a product.
 template <typename T, typename Cfg, int A_PLANES, typename Epi>
-__global__ void __launch_bounds__(Cfg::kThreads) __attribute__((amdgpu_waves_per_eu(1, EDHMC_GEMM_WPE)))
-gemm_nt_kernel(GemmShape g, Epi epi) {
+__device__ __forceinline__ void gemm_nt_tile(const GemmShape& g, const Epi& epi, int id) {
   constexpr int NT = Cfg::kThreads;
   constexpr int WM = Cfg::kWM, WN = Cfg::kWN, WAVES_M = Cfg::kWavesM;
   constexpr int BM = Cfg::BM, BN = Cfg::BN;
@@ -226,7 +226,7 @@ gemm_nt_kernel(GemmShape g, Epi epi) {
   __shared__ __align__(16) char smem[SMEM];
 
   int tm, tn, ks;
-  if (!map_tile(g, blockIdx.x, tm, tn, ks)) return;
+  if (!map_tile(g, id, tm, tn, ks)) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave % WAVES_M, wn = wave / WAVES_M;
   const int s_begin = ks * g.stages_per_split;
@@ -430,6 +430,12 @@ gemm_nt_kernel(GemmShape g, Epi epi) {
 #undef EDHMC_GLOAD
 
   EpiPre<Epi, Cfg>::apply(epi, acc, pos, pre);
+}
+
+template <typename T, typename Cfg, int A_PLANES, typename Epi>
+__global__ void __launch_bounds__(Cfg::kThreads) __attribute__((amdgpu_waves_per_eu(1, EDHMC_GEMM_WPE)))
+gemm_nt_kernel(GemmShape g, Epi epi) {
+  gemm_nt_tile<T, Cfg, A_PLANES>(g, epi, blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------

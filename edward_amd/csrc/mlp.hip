@@ -472,13 +472,29 @@ transpose_bf16_kernel(TransposeJob j0, TransposeJob j1) {
   for (int k = ty; k < 64; k += 4) jb.out[(int64_t)(c0 + k) * jb.R + r0 + tx] = t[tx][k];
 }
 
-// Row sums of a bf16 matrix [R x K] -> fp32 (bias gradients from transposed
-// activation gradients).  One wave per row, 16-byte loads (K is a multiple
-// of 128: the padded batch).
-__global__ void rowsum_bf16_kernel(const bf16_t* __restrict__ in, int R, int K, float* __restrict__ out) {
-  const int row = blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6);
+// Row sums of three bf16 matrices [R_i x K] -> fp32 (bias gradients from
+// transposed activation gradients).  One wave per row, 16-byte loads (K is a
+// multiple of 128: the padded batch).
+struct RowsumJobs {
+  const bf16_t* in[3];
+  float* out[3];
+  int R[3];
+};
+__global__ void rowsum_bf16_kernel(RowsumJobs jobs, int K) {
+  int row = blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  if (row >= R) return;
+  const bf16_t* in = jobs.in[0];
+  float* out = jobs.out[0];
+  if (row >= jobs.R[0] + jobs.R[1]) {
+    row -= jobs.R[0] + jobs.R[1];
+    in = jobs.in[2];
+    out = jobs.out[2];
+    if (row >= jobs.R[2]) return;
+  } else if (row >= jobs.R[0]) {
+    row -= jobs.R[0];
+    in = jobs.in[1];
+    out = jobs.out[1];
+  }
   float s = 0.0f;
   for (int k = 8 * lane; k < K; k += 512) {
     const uint4 v = *(const uint4*)(in + (int64_t)row * K + k);
@@ -639,6 +655,28 @@ static int mlp_gemm_cfg(edhmc_ctx* ctx, const void* A, int64_t lda_elems, const 
   return check_launch(ctx, "mlp_gemm");
 }
 
+// The three weight gradients of a training pass, each with few output tiles
+// and the batch as its long K, in one launch: 64 x 64 tiles leave one or less
+// of a product's per compute unit, two or more of all three.  Batch 4096, D =
+// 512, H = 1024: 45 us against three launches of 22 (128 x 64 tiles 47, 128 x
+// 128 43; row strides off the power of two change nothing).
+struct WeightGrads {
+  GemmShape g[3];
+  EpiStoreF32 e[3];
+  int first[3];   // workgroup each begins at
+};
+template <typename Cfg>
+__global__ void __launch_bounds__(Cfg::kThreads) __attribute__((amdgpu_waves_per_eu(1, EDHMC_GEMM_WPE)))
+weight_grads_kernel(WeightGrads w) {
+  const int b = blockIdx.x;
+  GemmShape g = w.g[0];
+  EpiStoreF32 e = w.e[0];
+  int first = 0;
+  if (b >= w.first[1]) { g = w.g[1]; e = w.e[1]; first = w.first[1]; }
+  if (b >= w.first[2]) { g = w.g[2]; e = w.e[2]; first = w.first[2]; }
+  gemm_nt_tile<bf16_t, Cfg, 1>(g, e, b - first);
+}
+
 // The tile shape by the number of 128 x 128 output tiles (M and N are
 // multiples of 128).  Measured on the 4096-chain layers (MI355X, us per
 // launch, 64 x 64 / chosen): 4096 x 1024 x 512  13.8 / 9.8,
@@ -652,6 +690,53 @@ static int mlp_gemm(edhmc_ctx* ctx, const void* A, int64_t lda_elems, const void
   if (tiles >= 256) return mlp_gemm_cfg<CfgM8>(ctx, A, lda_elems, B, ldb_elems, M, N, K, e, st);
   if (tiles >= 128) return mlp_gemm_cfg<CfgM8N>(ctx, A, lda_elems, B, ldb_elems, M, N, K, e, st);
   return mlp_gemm_cfg<CfgMS>(ctx, A, lda_elems, B, ldb_elems, M, N, K, e, st);
+}
+
+// out[i] = A_i B_i^T, all with K columns; M and N multiples of 128.
+struct WeightGrad {
+  const void* A; const void* B;
+  int M, N, ldc;
+  float* out;
+};
+static int weight_grads(edhmc_ctx* ctx, const WeightGrad (&job)[3], int K, hipStream_t st) {
+  int most = 0;
+  for (const WeightGrad& q : job) most = std::max(most, (q.M / 128) * (q.N / 128));
+  if (most >= 128) {   // (H = 1536 and more) mlp_gemm's larger tiles fill the chip
+    for (const WeightGrad& q : job) {
+      EpiStoreF32 e;
+      e.out = q.out;
+      e.ldc = q.ldc;
+      e.split_b = 0;
+      EDHMC_TRY(mlp_gemm(ctx, q.A, K, q.B, K, q.M, q.N, K, e, st));
+    }
+    return EDHMC_OK;
+  }
+  using Cfg = CfgMS;
+  WeightGrads w = {};
+  int at = 0;
+  for (int i = 0; i < 3; ++i) {
+    GemmShape& g = w.g[i];
+    g.A = (const char*)job[i].A;
+    g.B = (const char*)job[i].B;
+    g.lda_b = g.ldb_b = (int64_t)K * 2;
+    g.a_stage_b = g.b_stage_b = Cfg::KS;
+    g.m_tiles = job[i].M / Cfg::BM;
+    g.n_tiles = job[i].N / Cfg::BN;
+    g.k_stages = g.stages_per_split = K * 2 / Cfg::KS;
+    g.ksplit = 1;
+    if (job[i].M % Cfg::BM || job[i].N % Cfg::BN || (K * 2) % Cfg::KS)
+      return set_err(ctx, EDHMC_EUNSUPPORTED, "weight gradient %d x %d x %d does not fit the tiles",
+                     job[i].M, job[i].N, K);
+    if (!gemm_offsets_fit<Cfg, 1>(g)) return set_err(ctx, EDHMC_EUNSUPPORTED, "MLP tile too large");
+    w.e[i].out = job[i].out;
+    w.e[i].ldc = job[i].ldc;
+    w.e[i].split_b = 0;
+    w.first[i] = at;
+    at += grid_size(g);
+  }
+  ProfScope ps(ctx, PK_MLP, st);
+  hipLaunchKernelGGL((weight_grads_kernel<Cfg>), dim3(at), dim3(Cfg::kThreads), 0, st, w);
+  return check_launch(ctx, "weight_grads");
 }
 
 // One launch for one or two bf16 transposes (in [R x Cc] -> out [Cc x R]).
@@ -773,15 +858,6 @@ static int loss_grad(edhmc_ctx* ctx, Surrogate* s, const float* W, const float* 
   EDHMC_TRY(check_launch(ctx, "loss_sum"));
   if (!backward) return EDHMC_OK;   // the loss alone
   float* Gr = (float*)s->Gr.p;
-  // layer 3 weights: dW3 = dO^T [h2 | x0], db3 = column sums of dO
-  EpiStoreF32 ew;
-  ew.split_b = 0;
-  ew.out = Gr + s->oW3;
-  ew.ldc = s->Kc;
-  EDHMC_TRY(mlp_gemm(ctx, s->dOt.p, Bp, h2t, Bp, s->Dp, s->Kc, Bp, ew, st));
-  hipLaunchKernelGGL(rowsum_bf16_kernel, dim3(blocks_for(s->Dp, 4)), dim3(256), 0, st,
-                     (const bf16_t*)s->dOt.p, s->Dp, Bp, Gr + s->ob3);
-  EDHMC_TRY(check_launch(ctx, "rowsum"));
   // da2 = (dO W3) * GELU'(a2)
   EpiGeluBack eb2;
   eb2.a_in = (const float*)s->a2.p;
@@ -790,12 +866,6 @@ static int loss_grad(edhmc_ctx* ctx, Surrogate* s, const float* W, const float* 
   eb2.dat_out = (bf16_t*)s->da2t.p;
   eb2.ldt = Bp;
   EDHMC_TRY(mlp_gemm(ctx, s->dO.p, s->Dp, s->W3t.p, s->Dp, Bp, s->Hp, s->Dp, eb2, st));
-  ew.out = Gr + s->oW2;
-  ew.ldc = s->Hp;
-  EDHMC_TRY(mlp_gemm(ctx, s->da2t.p, Bp, s->h1t.p, Bp, s->Hp, s->Hp, Bp, ew, st));
-  hipLaunchKernelGGL(rowsum_bf16_kernel, dim3(blocks_for(s->Hp, 4)), dim3(256), 0, st,
-                     (const bf16_t*)s->da2t.p, s->Hp, Bp, Gr + s->ob2);
-  EDHMC_TRY(check_launch(ctx, "rowsum"));
   // da1 = (da2 W2) * GELU'(a1)
   EpiGeluBack eb1;
   eb1.a_in = (const float*)s->a1.p;
@@ -804,11 +874,18 @@ static int loss_grad(edhmc_ctx* ctx, Surrogate* s, const float* W, const float* 
   eb1.dat_out = (bf16_t*)s->da1t.p;
   eb1.ldt = Bp;
   EDHMC_TRY(mlp_gemm(ctx, s->da2.p, s->Hp, s->W2t.p, s->Hp, Bp, s->Hp, s->Hp, eb1, st));
-  ew.out = Gr + s->oW1;
-  ew.ldc = s->Dp;
-  EDHMC_TRY(mlp_gemm(ctx, s->da1t.p, Bp, x0t, Bp, s->Hp, s->Dp, Bp, ew, st));
-  hipLaunchKernelGGL(rowsum_bf16_kernel, dim3(blocks_for(s->Hp, 4)), dim3(256), 0, st,
-                     (const bf16_t*)s->da1t.p, s->Hp, Bp, Gr + s->ob1);
+  // weights: dW3 = dO^T [h2 | x0], dW2 = da2^T h1, dW1 = da1^T x0; biases:
+  // column sums of dO, da2, da1
+  const WeightGrad jobs[3] = {{s->dOt.p, h2t, s->Dp, s->Kc, s->Kc, Gr + s->oW3},
+                              {s->da2t.p, s->h1t.p, s->Hp, s->Hp, s->Hp, Gr + s->oW2},
+                              {s->da1t.p, x0t, s->Hp, s->Dp, s->Dp, Gr + s->oW1}};
+  EDHMC_TRY(weight_grads(ctx, jobs, Bp, st));
+  RowsumJobs rj;
+  rj.in[0] = (const bf16_t*)s->dOt.p; rj.out[0] = Gr + s->ob3; rj.R[0] = s->Dp;
+  rj.in[1] = (const bf16_t*)s->da2t.p; rj.out[1] = Gr + s->ob2; rj.R[1] = s->Hp;
+  rj.in[2] = (const bf16_t*)s->da1t.p; rj.out[2] = Gr + s->ob1; rj.R[2] = s->Hp;
+  hipLaunchKernelGGL(rowsum_bf16_kernel, dim3(blocks_for(s->Dp + 2 * s->Hp, 4)), dim3(256), 0, st,
+                     rj, Bp);
   return check_launch(ctx, "rowsum");
 }
 
