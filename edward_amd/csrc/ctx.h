@@ -134,6 +134,7 @@ struct edhmc_ctx {
   edhmc::DevBuf ll_split;   // log-likelihood range sums [16][C_pad] (fixed-order reduction)
   edhmc::DevBuf newton;          // scratch of edhmc_newton_terms
   edhmc::DevBuf acov_part, acov_mean;   // autocovariance partial sums, chain means
+  edhmc::DevBuf eta;   // one-pass gradient: eta of rows whose log-likelihood has its own kernel
   edhmc::DevBuf acov_rows, acov, ess_spread;   // transposed chains; all lags; spread of the means
 
   edhmc::Profiler prof;

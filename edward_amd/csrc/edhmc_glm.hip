@@ -1231,7 +1231,7 @@ static int rows_eval(edhmc_ctx* ctx, bool ll, hipStream_t st, const HierRows* hr
   a.g_ld = ctx->g_ld;
   a.llpart = (double*)ctx->llpart.p;
   a.ll_ld = ctx->C_pad;
-  a.eta = (float*)ctx->Rt.p;
+  a.eta = (float*)ctx->eta.p;
   if (hr) {
     a.goff = hr->goff;
     a.goff_ld = hr->goff_ld;
@@ -1283,21 +1283,14 @@ static int grad_eval(edhmc_ctx* ctx, bool split, bool ll, hipStream_t st) {
 #ifndef EDHMC_CFG_H
 #define EDHMC_CFG_H 2, 2, 2, 2, 128
 #endif
-// GEMM1 of the hierarchical model (its log-likelihood, and its residuals
-// where D_pad > 256): 128-byte K stages, half the stage barriers (1.11 vs
-// 1.19 ms at G = 2048, D = 64, 512 chains)
+// GEMM1 of the hierarchical model where D_pad > 256: 128-byte K stages, half
+// the stage barriers
 using CfgH = TileCfg<EDHMC_CFG_H>;
 int glm_grad_eval_offset(edhmc_ctx* ctx, const HierRows& hr, bool ll, hipStream_t st,
                          int64_t* summed_rows) {
   *summed_rows = 0;
   if (ctx->cdt != EDHMC_F32) return set_err(ctx, EDHMC_EUNSUPPORTED, "offset path is fp32");
-  if (rows_ok(ctx)) {
-    EDHMC_TRY(rows_eval(ctx, false, st, &hr, summed_rows));
-    // the log-likelihood in GEMM1's forward form: its FP64 partial sums keep
-    // their order over the rows
-    return ll ? launch_gemm1<float, CfgH, 1, false, true>(ctx, st, hr.goff, hr.goff_ld, hr.gidx)
-              : EDHMC_OK;
-  }
+  if (rows_ok(ctx)) return rows_eval(ctx, ll, st, &hr, summed_rows);
   if (ctx->C_pad % CfgH::BM || ctx->N_pad % CfgH::BN)
     return set_err(ctx, EDHMC_EUNSUPPORTED, "hierarchical GEMM1 tiles do not divide the padding");
   if (ll) EDHMC_TRY((launch_gemm1<float, CfgH, 1, true, true>(ctx, st, hr.goff, hr.goff_ld, hr.gidx)));
@@ -2058,14 +2051,13 @@ static int ensure_chains(edhmc_ctx* ctx, int C, hipStream_t st) {
     if (ks >= 8) ks = ks / 8 * 8;
     ctx->ksplit = ks;
     ctx->g_ld = C_pad;
-    // residuals, or after a one-pass gradient (but the hierarchical model's)
-    // eta of the rows whose log-likelihood is summed in a kernel of its own;
+    // residuals: none after a one-pass gradient but the hierarchical model's;
     // rows up to a whole W-stationary tile, whose residual epilogue stores the
     // last tile's rows past N_pad (zeros) without a bounds test
-    const size_t rt = rows_ok(ctx) && !ctx->hier
-                          ? (size_t)rows_eta(C, ks, ctx->N_pad) * 4
-                          : (size_t)C_pad * round_up(ctx->N_pad, kWsTile) * eb;
-    EDHMC_TRY(dev_alloc(ctx, ctx->Rt, rt, false));
+    if (rows_ok(ctx)) EDHMC_TRY(dev_alloc(ctx, ctx->eta, (size_t)rows_eta(C, ks, ctx->N_pad) * 4, false));
+    else ctx->eta.release();
+    if (rows_ok(ctx) && !ctx->hier) ctx->Rt.release();
+    else EDHMC_TRY(dev_alloc(ctx, ctx->Rt, (size_t)C_pad * round_up(ctx->N_pad, kWsTile) * eb, false));
   }
   EDHMC_TRY(dev_alloc(ctx, ctx->Gpart, (size_t)ctx->ksplit * ctx->g_ld * ctx->D_pad * 4, false));
   EDHMC_TRY(dev_alloc(ctx, ctx->llpart, (size_t)C_pad * ctx->n_tiles1 * 8, false));
@@ -2268,7 +2260,7 @@ edhmc_ctx::~edhmc_ctx() {
   DevBuf* bufs[] = {&Xr, &Xc, &Xf, &Xs, &Xp, &yp, &y, &ploc, &pscale, &z, &r, &g, &z0, &g0, &z_lp, &logp, &K0,
                     &flag, &ndiv, &ratio, &Rt, &Gpart, &llpart, &ll, &mom_mean, &mom_m2, &tmp_count,
                     &stats_part, &pred_col, &ll_split, &pkind, &plnorm,
-                    &newton, &acov_part, &acov_mean, &acov_rows, &acov, &ess_spread};
+                    &newton, &eta, &acov_part, &acov_mean, &acov_rows, &acov, &ess_spread};
   for (DevBuf* b : bufs) b->release();
 }
 

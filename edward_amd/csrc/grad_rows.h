@@ -295,10 +295,14 @@ grad_rows_kernel(RowsArgs a) {
     for (int b = 0; b < RB; ++b) {
       const int blk = rw * RB + b;
       f32x4_t r;
+      if (HIER) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) e[b][v] = e[b][v] + oc[b][v];
+      }
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const bool ok = 16 * blk + pi16(4 * h + v) < left;
-        const float eta = HIER ? e[b][v] + oc[b][v] : e[b][v];
+        const float eta = e[b][v];
         r[v] = ok ? glm_dll(lp, eta, yc[b][v]) : 0.0f;
       }
       if (LL && 16 * blk < left) {   // not a block of the next range
@@ -588,6 +592,10 @@ grad_wide_kernel(RowsArgs a) {
   // residuals of block b of tile t, in place
   auto residual = [&](int t, f32x4_t (&e)[RB], int b) {
     const int64_t nb = n0 + (int64_t)t * TR + 16 * b;
+    if (HIER) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) e[b][v] = e[b][v] + oc[b][v];
+    }
     bool here = false;    // its 128-row tile lies within this range
     if (LL && nb < n_end) {
       const int64_t tb = nb / kLLTile * kLLTile;
@@ -600,7 +608,7 @@ grad_wide_kernel(RowsArgs a) {
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const bool ok = t * TR + 16 * b + pi16(4 * h + v) < rows;
-      const float eta = HIER ? e[b][v] + oc[b][v] : e[b][v];
+      const float eta = e[b][v];
       float dll;
       if (LL) {
         double ll;

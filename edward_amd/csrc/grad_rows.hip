@@ -34,7 +34,8 @@ static void launch_cw(RowsArgs a, bool ll, hipStream_t st) {
   a.tiles = (a.C + 16 * CW - 1) / (16 * CW);
   const dim3 grid(a.tiles * a.splits), block(256);
   const bool bern = a.lp.lik == LIK_BERNOULLI;
-  if (a.goff) hipLaunchKernelGGL((grad_rows_kernel<DP, CW, false, true, true>), grid, block, 0, st, a);
+  if (a.goff && ll) hipLaunchKernelGGL((grad_rows_kernel<DP, CW, true, true, true>), grid, block, 0, st, a);
+  else if (a.goff) hipLaunchKernelGGL((grad_rows_kernel<DP, CW, false, true, true>), grid, block, 0, st, a);
   else if (bern && ll) hipLaunchKernelGGL((grad_rows_kernel<DP, CW, true, false, true>), grid, block, 0, st, a);
   else if (bern) hipLaunchKernelGGL((grad_rows_kernel<DP, CW, false, false, true>), grid, block, 0, st, a);
   else if (ll) hipLaunchKernelGGL((grad_rows_kernel<DP, CW, true, false, false>), grid, block, 0, st, a);
@@ -46,7 +47,8 @@ static void launch_wide(RowsArgs a, bool ll, hipStream_t st) {
   a.tiles = (a.C + 63) / 64;
   const dim3 grid(a.tiles * a.splits), block(256);
   const bool bern = a.lp.lik == LIK_BERNOULLI;
-  if (a.goff) hipLaunchKernelGGL((grad_wide_kernel<DP, false, true, true>), grid, block, 0, st, a);
+  if (a.goff && ll) hipLaunchKernelGGL((grad_wide_kernel<DP, true, true, true>), grid, block, 0, st, a);
+  else if (a.goff) hipLaunchKernelGGL((grad_wide_kernel<DP, false, true, true>), grid, block, 0, st, a);
   else if (bern && ll) hipLaunchKernelGGL((grad_wide_kernel<DP, true, false, true>), grid, block, 0, st, a);
   else if (bern) hipLaunchKernelGGL((grad_wide_kernel<DP, false, false, true>), grid, block, 0, st, a);
   else if (ll) hipLaunchKernelGGL((grad_wide_kernel<DP, true, false, false>), grid, block, 0, st, a);
