@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace edhmc {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
@@ -76,6 +78,29 @@ __device__ inline double block_sum_f64(double v, double* sm /* >= NT/64 */) {
 #pragma unroll
   for (int w = 0; w < NT / 64; ++w) t += sm[w];
   return t;
+}
+
+// Sum of p[q * stride], q < n, in order: sixteen loads in flight, then eight
+// (n is a multiple of 8 from 8 on in the gradient's partial sums), four, one.
+// A loop unrolled sixteen times took the eight of a small model one by one: 390
+// chains on 2507 x 193, bf16, 498 us a transition of eleven steps, here 480.
+__device__ inline float strided_sum(const float* p, int64_t stride, int n) {
+  float s = 0.0f;
+  int q = 0;
+  auto add = [&](auto count) {
+    constexpr int K = decltype(count)::value;
+    float v[K];
+#pragma unroll
+    for (int i = 0; i < K; ++i) v[i] = p[(q + i) * stride];
+#pragma unroll
+    for (int i = 0; i < K; ++i) s += v[i];
+    q += K;
+  };
+  while (q + 16 <= n) add(std::integral_constant<int, 16>{});
+  if (q + 8 <= n) add(std::integral_constant<int, 8>{});
+  if (q + 4 <= n) add(std::integral_constant<int, 4>{});
+  while (q < n) add(std::integral_constant<int, 1>{});
+  return s;
 }
 
 // ---------------------------------------------------------------------------

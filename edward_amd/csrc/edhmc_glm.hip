@@ -602,11 +602,7 @@ __global__ void __launch_bounds__(kChainThreads) chain_begin_kernel(ChainArgs a)
 }
 
 __device__ inline float gsum(const ChainArgs& a, int c, int d) {
-  const float* p = a.Gpart + (int64_t)c * a.D_pad + d;
-  float s = 0.0f;
-#pragma unroll 16
-  for (int q = 0; q < a.ksplit; ++q) s += p[q * a.g_stride];
-  return a.lik_weight * s;
+  return a.lik_weight * strided_sum(a.Gpart + (int64_t)c * a.D_pad + d, a.g_stride, a.ksplit);
 }
 
 // The likelihood gradient of chain c for every coordinate, by the whole

@@ -164,9 +164,7 @@ __device__ inline void hier_assemble(const HierArgs& a, int c, bool want_lp, dou
     } else {
       const int d = j - a.G - 2;
       const float* gp = a.Gpart + (int64_t)c * a.D_pad + d;
-      float s = 0.0f;
-#pragma unroll 16
-      for (int q = 0; q < a.ksplit; ++q) s += gp[q * gstride];
+      const float s = strided_sum(gp, gstride, a.ksplit);
       gv = s - th[j];
     }
     g[j] = gv;
