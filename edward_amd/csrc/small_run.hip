@@ -37,7 +37,9 @@ small_run_kernel(SmallArgs a) {
   static_assert(XB <= kSmallRegs && 64 % DP == 0, "registers");
   __shared__ __align__(16) float rs[RPT * kSmallThreads];
   __shared__ float red[kSmallWaves][DP];
-  __shared__ double dsum[kSmallWaves];
+  // by the parity of the transition: with one step a transition, a wave may be
+  // at the next one's sum while another still reads this one's
+  __shared__ double dsum[2][kSmallWaves];
   const int c = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int d = lane % DP;
@@ -73,6 +75,7 @@ small_run_kernel(SmallArgs a) {
   int n_acc = 0, n_div = 0, acc = 0;
   for (int t = 0; t < a.T; ++t) {
     const uint64_t counter = a.counter + (uint64_t)t;
+    double* const ds = dsum[t & 1];
     z0 = z;
     g0 = g;
     r = 0.0f;
@@ -117,7 +120,7 @@ small_run_kernel(SmallArgs a) {
       }
       if (last) {
         lls = wave_sum_f64(lls);
-        if (lane == 0) dsum[wave] = lls;
+        if (lane == 0) ds[wave] = lls;
       }
       __syncthreads();
       float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -139,7 +142,7 @@ small_run_kernel(SmallArgs a) {
       r = r + a.half * g;
       if (last) {
 #pragma unroll
-        for (int w = 0; w < kSmallWaves; ++w) ll += dsum[w];
+        for (int w = 0; w < kSmallWaves; ++w) ll += ds[w];
       } else {
         r = r + a.half * g;
         z = z + a.full * r;
