@@ -134,6 +134,7 @@ struct edhmc_ctx {
   edhmc::DevBuf ll_split;   // log-likelihood range sums [16][C_pad] (fixed-order reduction)
   edhmc::DevBuf newton;          // scratch of edhmc_newton_terms
   edhmc::DevBuf acov_part, acov_mean;   // autocovariance partial sums, chain means
+  hipEvent_t acov_used = nullptr;       // end of the last readout call with this scratch
   edhmc::DevBuf eta;   // one-pass gradient: eta of rows whose log-likelihood has its own kernel
   edhmc::DevBuf acov_rows, acov, ess_spread;   // transposed chains; all lags; spread of the means
 
@@ -198,6 +199,12 @@ inline int check_launch(edhmc_ctx* ctx, const char* what) {
   if (e != hipSuccess)
     return set_err(ctx, EDHMC_EHIP, "%s: %s", what, hipGetErrorString(e));
   return EDHMC_OK;
+}
+
+inline bool stream_capturing(hipStream_t st) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &cap) != hipSuccess) (void)hipGetLastError();
+  return cap != hipStreamCaptureStatusNone;
 }
 
 inline int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }

@@ -2258,6 +2258,7 @@ edhmc_ctx::~edhmc_ctx() {
                     &stats_part, &pred_col, &ll_split, &pkind, &plnorm,
                     &newton, &eta, &acov_part, &acov_mean, &acov_rows, &acov, &ess_spread};
   for (DevBuf* b : bufs) b->release();
+  if (acov_used) (void)hipEventDestroy(acov_used);
 }
 
 extern "C" {

@@ -131,7 +131,9 @@ int launch_moments(edhmc_ctx* ctx, const P* x, int64_t T, int64_t K, int64_t t0,
 // for the loads.  T = 1000, C = 1024, D = 256, all 1000 lags in five windows:
 // 14.8 ms, against 105 ms for a thread per series with one atomic per series
 // and lag.  It takes windows that do not begin at lag 0, at most 32 lags, and
-// more than 2048 draws (acov_fft.hip the others).
+// more than 2048 draws (acov_fft.hip the others), and whatever has to do
+// without scratch: then one group, chains one after the other, its sums
+// straight in the output, and with OWN_MEAN the chain means made here.
 // ---------------------------------------------------------------------------
 constexpr int kAcLags = 32, kAcStep = 8, kAcWaves = 4;
 constexpr int kAcWin = kAcLags / kAcStep + 1;   // window of kAcWin kAcStep values
@@ -143,10 +145,11 @@ struct AcovArgs {
   int lag0, n_lags;
   int blocks, groups;      // chain blocks of m chains, groups of them
   int strips, lag_wgs;     // 64-column strips of P, workgroups along the lags
-  const double* mean;      // [C][D]
+  const double* mean;      // [C][D] (OWN_MEAN: not read)
   double* part;            // [groups][n_lags][P]
 };
 
+template <bool OWN_MEAN>
 __global__ void __launch_bounds__(64 * kAcWaves) __attribute__((amdgpu_waves_per_eu(1, 2)))
 autocov_kernel(AcovArgs a) {
   // units (strip, chain group) dealt to the XCDs, all lags of a unit on one
@@ -176,7 +179,15 @@ autocov_kernel(AcovArgs a) {
     if (v >= a.P || c >= a.C) continue;
     const float* p = a.s + (int64_t)k * a.m * a.D;   // row of draw 0; the lane reads column v
     auto x_at = [&](int64_t t) -> float { return (p + min(t, T - 1) * stride)[(uint32_t)v]; };
-    const double mean = a.mean[(int64_t)c * a.D + d];
+    double mean;
+    if constexpr (OWN_MEAN) {
+      mean = 0.0;
+#pragma unroll 16
+      for (int64_t t = 0; t < T; ++t) mean += (double)x_at(t);
+      mean /= (double)T;
+    } else {
+      mean = a.mean[(int64_t)c * a.D + d];
+    }
     double w[kAcWin][kAcStep];
     // a_t at times past the last draw read as 0
 #pragma unroll
@@ -233,10 +244,11 @@ autocov_kernel(AcovArgs a) {
       a.part[((int64_t)grp * a.n_lags + lb * kAcLags + l) * a.P + v] = acc[l];
 }
 
-// acov[l][d] = sum over the groups and the m side-by-side chains, / T.
+// acov[l][d] = sum over the groups and the m side-by-side chains, / T (in place
+// where both are 1 and acov is part).
 __global__ void __launch_bounds__(256)
-autocov_sum_kernel(const double* __restrict__ part, int groups, int n_lags, int m, int D, int64_t T,
-                   double* __restrict__ acov) {
+autocov_sum_kernel(const double* part, int groups, int n_lags, int m, int D, int64_t T,
+                   double* acov) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= (int64_t)n_lags * D) return;
   const int64_t l = i / D;
@@ -248,35 +260,48 @@ autocov_sum_kernel(const double* __restrict__ part, int groups, int n_lags, int 
   acov[i] = s / (double)T;
 }
 
+// scratch: whether the context's may be used (and grow); without it, and where
+// the device has no memory for it, the call does without.
 int autocov_lags(edhmc_ctx* ctx, const float* s, int64_t T, int C, int D, int lag0, int n_lags,
-                 const double* mean, double* acov, hipStream_t st) {
+                 const double* mean, double* acov, bool scratch, hipStream_t st) {
   AcovArgs a;
   a.s = s;
   a.T = T;
   a.C = C;
   a.D = D;
-  a.m = std::max(1, std::min(C, 64 / D));
-  a.P = D * a.m;
   a.lag0 = lag0;
   a.n_lags = n_lags;
-  a.blocks = (C + a.m - 1) / a.m;
-  a.strips = (a.P + 63) / 64;
+  a.mean = mean;
   const int lag_blocks = (n_lags + kAcLags - 1) / kAcLags;
   a.lag_wgs = (lag_blocks + kAcWaves - 1) / kAcWaves;
+  auto split = [&](int m, int64_t most) {   // m chains side by side, at most that many groups
+    a.m = m;
+    a.P = D * m;
+    a.blocks = (C + m - 1) / m;
+    a.strips = (a.P + 63) / 64;
+    const int64_t groups = std::min<int64_t>(most, a.blocks);
+    const int64_t per = (a.blocks + groups - 1) / groups;
+    a.groups = (int)((a.blocks + per - 1) / per);
+  };
+  const int m = std::max(1, std::min(C, 64 / D));
   // eight rounds of the 2048 waves that run together, so that the shorter
   // sums of the long lags even out; at most 128 MB of partial sums
-  int64_t groups = std::max<int64_t>(1, 16384 / ((int64_t)a.strips * a.lag_wgs * kAcWaves));
-  groups = std::min<int64_t>(groups, std::max<int64_t>(1, (128 << 20) / ((int64_t)n_lags * a.P * 8)));
-  groups = std::min<int64_t>(groups, a.blocks);
-  const int64_t per = (a.blocks + groups - 1) / groups;
-  a.groups = (int)((a.blocks + per - 1) / per);
-  a.mean = mean;
-  EDHMC_TRY(dev_reserve(ctx, ctx->acov_part, (size_t)a.groups * n_lags * a.P * 8));
-  a.part = (double*)ctx->acov_part.p;
+  const int64_t strips = ((int64_t)D * m + 63) / 64;
+  int64_t groups = std::max<int64_t>(1, 16384 / (strips * a.lag_wgs * kAcWaves));
+  groups = std::min<int64_t>(groups, std::max<int64_t>(1, (128 << 20) / ((int64_t)n_lags * D * m * 8)));
+  split(m, groups);
+  if (scratch && dev_reserve(ctx, ctx->acov_part, (size_t)a.groups * n_lags * a.P * 8) == EDHMC_OK) {
+    a.part = (double*)ctx->acov_part.p;
+  } else {
+    split(1, 1);
+    a.part = acov;
+  }
   const int64_t units = (int64_t)a.strips * a.groups;
   const int64_t grid = (units + 7) / 8 * 8 * a.lag_wgs;
   if (grid > 2147483647LL) return set_err(ctx, EDHMC_EUNSUPPORTED, "autocov: store too wide");
-  hipLaunchKernelGGL(autocov_kernel, dim3((unsigned)grid), dim3(64 * kAcWaves), 0, st, a);
+  const dim3 wgs((unsigned)grid), block(64 * kAcWaves);
+  if (mean) hipLaunchKernelGGL(autocov_kernel<false>, wgs, block, 0, st, a);
+  else hipLaunchKernelGGL(autocov_kernel<true>, wgs, block, 0, st, a);
   EDHMC_TRY(check_launch(ctx, "autocov"));
   const int64_t n = (int64_t)n_lags * D;
   hipLaunchKernelGGL(autocov_sum_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
@@ -284,13 +309,46 @@ int autocov_lags(edhmc_ctx* ctx, const float* s, int64_t T, int C, int D, int la
   return check_launch(ctx, "autocov_sum");
 }
 
-// Lags 0 .. n_lags - 1 and the chain means they take.
+// Lags 0 .. n_lags - 1 and, if asked for, the chain means they take.
 int autocov_from_zero(edhmc_ctx* ctx, const float* s, int64_t T, int C, int D, int n_lags,
-                      double* mean, double* acov, hipStream_t st) {
-  if (autocov_fft_ok(T, n_lags)) return autocov_fft(ctx, s, T, C, D, n_lags, mean, acov, st);
-  EDHMC_TRY(launch_moments<float>(ctx, s, T, (int64_t)C * D, 0, mean, nullptr, st));
-  return autocov_lags(ctx, s, T, C, D, 0, n_lags, mean, acov, st);
+                      double* mean, double* acov, bool scratch, hipStream_t st) {
+  if (!mean && scratch && dev_reserve(ctx, ctx->acov_mean, (size_t)C * D * 8) == EDHMC_OK)
+    mean = (double*)ctx->acov_mean.p;
+  if (mean && scratch && autocov_fft_ok(T, n_lags)) {
+    const int rc = autocov_fft(ctx, s, T, C, D, n_lags, mean, acov, st);
+    if (rc != EDHMC_ENOMEM) return rc;   // (before it has launched anything)
+  }
+  if (mean) EDHMC_TRY(launch_moments<float>(ctx, s, T, (int64_t)C * D, 0, mean, nullptr, st));
+  return autocov_lags(ctx, s, T, C, D, 0, n_lags, mean, acov, scratch, st);
 }
+
+// A call's turn with the context's readout scratch: it begins when the call
+// before has ended, on whatever stream that runs.  Under capture there is none:
+// the graph would keep the address of memory that later calls write and grow.
+struct ScratchTurn {
+  edhmc_ctx* ctx;
+  hipStream_t st;
+  bool on = false;
+
+  int begin() {
+    if (stream_capturing(st)) return EDHMC_OK;
+    if (!ctx->acov_used &&
+        hipEventCreateWithFlags(&ctx->acov_used, hipEventDisableTiming) != hipSuccess) {
+      (void)hipGetLastError();
+      ctx->acov_used = nullptr;
+      return set_err(ctx, EDHMC_EHIP, "readout: event");
+    }
+    if (hipStreamWaitEvent(st, ctx->acov_used, 0) != hipSuccess)
+      return set_err(ctx, EDHMC_EHIP, "readout: wait");
+    on = true;
+    return EDHMC_OK;
+  }
+  int end(int rc) {   // also after an error: something may be running
+    if (on && hipEventRecord(ctx->acov_used, st) != hipSuccess && rc == EDHMC_OK)
+      return set_err(ctx, EDHMC_EHIP, "readout: event");
+    return rc;
+  }
+};
 
 }  // namespace
 
@@ -326,13 +384,10 @@ int edhmc_autocov(edhmc_ctx* ctx, const float* s, int64_t T, int32_t C, int32_t 
   if (!s || !acov_out || T < 2 || C <= 0 || D <= 0 || max_lag < 0)
     return set_err(ctx, EDHMC_EINVAL, "bad arguments");
   if (max_lag >= T) max_lag = (int)(T - 1);
-  const int64_t K = (int64_t)C * D;
-  double* mean = chain_mean_out;
-  if (!mean) {
-    EDHMC_TRY(dev_reserve(ctx, ctx->acov_mean, (size_t)K * 8));
-    mean = (double*)ctx->acov_mean.p;
-  }
-  return autocov_from_zero(ctx, s, T, C, D, max_lag + 1, mean, acov_out, st);
+  ScratchTurn turn{ctx, st};
+  EDHMC_TRY(turn.begin());
+  return turn.end(autocov_from_zero(ctx, s, T, C, D, max_lag + 1, chain_mean_out, acov_out, turn.on,
+                                    st));
 }
 
 int edhmc_ess(edhmc_ctx* ctx, const float* s, int64_t T, int32_t C, int32_t D, int32_t between,
@@ -342,12 +397,18 @@ int edhmc_ess(edhmc_ctx* ctx, const float* s, int64_t T, int32_t C, int32_t D, i
   hipStream_t st = (hipStream_t)stream;
   if (!s || !ess_out || T < 4 || T > 2147483647LL || C <= 0 || D <= 0)
     return set_err(ctx, EDHMC_EINVAL, "bad arguments");
-  EDHMC_TRY(dev_reserve(ctx, ctx->acov_mean, (size_t)C * D * 8));
-  EDHMC_TRY(dev_reserve(ctx, ctx->acov, (size_t)T * D * 8));
-  double* mean = (double*)ctx->acov_mean.p;
-  double* acov = (double*)ctx->acov.p;
-  EDHMC_TRY(autocov_from_zero(ctx, s, T, C, D, (int)T, mean, acov, st));
-  return ess_launch(ctx, acov, mean, T, C, D, between != 0, ess_out, st);
+  ScratchTurn turn{ctx, st};
+  EDHMC_TRY(turn.begin());
+  if (!turn.on) return set_err(ctx, EDHMC_EUNSUPPORTED, "edhmc_ess cannot be captured in a graph");
+  auto go = [&]() -> int {
+    EDHMC_TRY(dev_reserve(ctx, ctx->acov_mean, (size_t)C * D * 8));
+    EDHMC_TRY(dev_reserve(ctx, ctx->acov, (size_t)T * D * 8));
+    double* mean = (double*)ctx->acov_mean.p;
+    double* acov = (double*)ctx->acov.p;
+    EDHMC_TRY(autocov_from_zero(ctx, s, T, C, D, (int)T, mean, acov, true, st));
+    return ess_launch(ctx, acov, mean, T, C, D, between != 0, ess_out, st);
+  };
+  return turn.end(go());
 }
 
 int edhmc_autocov_lags(edhmc_ctx* ctx, const float* s, int64_t T, int32_t C, int32_t D,
@@ -358,7 +419,10 @@ int edhmc_autocov_lags(edhmc_ctx* ctx, const float* s, int64_t T, int32_t C, int
   if (!s || !acov_out || !chain_mean || T < 2 || C <= 0 || D <= 0 || lag0 < 0 || n_lags <= 0 ||
       (int64_t)lag0 + n_lags > T)
     return set_err(ctx, EDHMC_EINVAL, "bad arguments");
-  return autocov_lags(ctx, s, T, C, D, lag0, n_lags, chain_mean, acov_out, (hipStream_t)stream);
+  ScratchTurn turn{ctx, (hipStream_t)stream};
+  EDHMC_TRY(turn.begin());
+  return turn.end(autocov_lags(ctx, s, T, C, D, lag0, n_lags, chain_mean, acov_out, turn.on,
+                               (hipStream_t)stream));
 }
 
 }  // extern "C"

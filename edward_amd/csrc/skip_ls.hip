@@ -211,9 +211,7 @@ int skip_gram(edhmc_ctx* ctx, DevBuf& scratch, hipEvent_t& used, const float* W,
   int splits = std::max(1, std::min(1024 / blocks, (n + 127) / 128));
   a.rows_per = ((n + splits - 1) / splits + 31) / 32 * 32;
   splits = (n + a.rows_per - 1) / a.rows_per;
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(st, &cap) != hipSuccess) (void)hipGetLastError();
-  if (splits > 1 && cap == hipStreamCaptureStatusNone &&
+  if (splits > 1 && !stream_capturing(st) &&
       (used || hipEventCreateWithFlags(&used, hipEventDisableTiming) == hipSuccess) &&
       hipStreamWaitEvent(st, used, 0) == hipSuccess &&
       dev_reserve(ctx, scratch, (size_t)splits * blocks * 4096 * 8) == EDHMC_OK) {

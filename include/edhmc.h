@@ -326,7 +326,12 @@ int edhmc_draw_uniforms(edhmc_ctx* ctx, int32_t C, uint64_t seed, uint64_t count
  * sample store s [T, C, D] fp32 (no reference counterpart; build-only):
  *   acov_out   [max_lag+1, D] fp64  sum over chains of the biased (/T)
  *              within-chain autocovariance at each lag
- *   chain_mean [C, D] fp64 (may be NULL to skip)                            */
+ *   chain_mean [C, D] fp64 (may be NULL to skip)
+ * This call and the two below share scratch that the context keeps: calls on
+ * several streams take turns with it (each waits on the device for the one
+ * before).  In a stream capture the two autocovariance calls do without, one
+ * group of chains after the other, as they do where the device has no memory
+ * for it; edhmc_ess refuses a capturing stream (EDHMC_EUNSUPPORTED).        */
 int edhmc_autocov(edhmc_ctx* ctx, const float* s, int64_t T, int32_t C, int32_t D,
                   int32_t max_lag, double* acov_out, double* chain_mean_out,
                   void* stream);
