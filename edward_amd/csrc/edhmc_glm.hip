@@ -2001,9 +2001,7 @@ static int launch_predict(edhmc_ctx* ctx, int S, bool want_mean, float* rep, uin
   return EDHMC_OK;
 }
 
-static int ensure_chains(edhmc_ctx* ctx, int C, hipStream_t st) {
-  if (C <= 0) return set_err(ctx, EDHMC_EINVAL, "number of chains must be positive, got %d", C);
-  if (ctx->C == C && ctx->z.p) return EDHMC_OK;
+static int alloc_chains(edhmc_ctx* ctx, int C, hipStream_t st) {
   const int C_pad = (int)round_up(C, kChainPad);
   const size_t cd = (size_t)C * ctx->D_pad;
   const int eb = elem_bytes(ctx);
@@ -2060,6 +2058,20 @@ static int ensure_chains(edhmc_ctx* ctx, int C, hipStream_t st) {
   EDHMC_TRY(dev_alloc(ctx, ctx->ll, (size_t)C_pad * 8));
   EDHMC_TRY(dev_alloc(ctx, ctx->ll_split, (size_t)kLLSplit * C_pad * 8, false));
   return EDHMC_OK;
+}
+
+// C and z.p say that all of a chain count's buffers are there: after a failure
+// there are no chains, and the next call starts over.
+static int ensure_chains(edhmc_ctx* ctx, int C, hipStream_t st) {
+  if (C <= 0) return set_err(ctx, EDHMC_EINVAL, "number of chains must be positive, got %d", C);
+  if (ctx->C == C && ctx->z.p) return EDHMC_OK;
+  const int rc = alloc_chains(ctx, C, st);
+  if (rc != EDHMC_OK) {
+    ctx->C = 0;
+    ctx->z.release();
+    ctx->Xs.release();
+  }
+  return rc;
 }
 
 int glm_ensure_chains(edhmc_ctx* ctx, int C, hipStream_t st) { return ensure_chains(ctx, C, st); }

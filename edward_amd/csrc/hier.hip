@@ -353,8 +353,10 @@ static int hier_set_state(edhmc_ctx* ctx, const float* theta, int C, hipStream_t
   HierModel* h = ctx->hier;
   if (!h) return set_err(ctx, EDHMC_ESTATE, "no hierarchical model bound");
   if (!theta) return set_err(ctx, EDHMC_EINVAL, "theta is NULL");
+  h->state_valid = false;
   EDHMC_TRY(glm_ensure_chains(ctx, C, st));
   if (h->C != C || h->C_pad != ctx->C_pad) {
+    h->C = 0;   // until all of them are there
     const size_t b = (size_t)ctx->C_pad * h->dim_pad * 4;
     EDHMC_TRY(dev_alloc(ctx, h->th, b));
     EDHMC_TRY(dev_alloc(ctx, h->r, b));
@@ -376,10 +378,7 @@ static int hier_set_state(edhmc_ctx* ctx, const float* theta, int C, hipStream_t
   if (hipMemcpyAsync(&bad, ctx->tmp_count.p, 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
       hipStreamSynchronize(st) != hipSuccess)
     return set_err(ctx, EDHMC_EHIP, "hier set_state: copy failed");
-  if (bad) {
-    h->state_valid = false;
-    return set_err(ctx, EDHMC_ENONFINITE, "theta contains %d non-finite rows", bad);
-  }
+  if (bad) return set_err(ctx, EDHMC_ENONFINITE, "theta contains %d non-finite rows", bad);
   EDHMC_TRY(hier_grad(ctx, h, true, st));
   hipLaunchKernelGGL(hier_eval_kernel, dim3(C), dim3(kHT), 0, st, a);
   EDHMC_TRY(check_launch(ctx, "hier_eval"));
@@ -427,6 +426,43 @@ static int hier_transition(edhmc_ctx* ctx, float eps, int L, const float* r0, co
 
 }  // namespace edhmc
 
+namespace edhmc {
+
+// The data of a new model in ctx->hier.
+static int hier_bind_data(edhmc_ctx* ctx, const float* X, const float* y, const int64_t* offsets,
+                          int G, int64_t N, int D, hipStream_t st) {
+  HierModel* h = new (std::nothrow) HierModel();
+  if (!h) return set_err(ctx, EDHMC_ENOMEM, "host allocation");
+  ctx->hier = h;
+  h->G = G;
+  h->D = D;
+  h->N = N;
+  h->dim = G + 2 + D;
+  h->dim_pad = (int)round_up(h->dim, 4);
+  // w ~ N(0, I): the GLM prior for the shared coefficients
+  EDHMC_TRY(dev_alloc(ctx, h->ones, (size_t)D * 4, false));
+  EDHMC_TRY(dev_alloc(ctx, h->zeros, (size_t)D * 4));
+  std::vector<float> one(D, 1.0f);
+  if (hipMemcpyAsync(h->ones.p, one.data(), (size_t)D * 4, hipMemcpyHostToDevice, st) != hipSuccess)
+    return set_err(ctx, EDHMC_EHIP, "copy");
+  EDHMC_TRY(edhmc_bind_glm(ctx, X, EDHMC_F32, y, N, D, EDHMC_LIK_BERNOULLI, 1.0f,
+                           (const float*)h->zeros.p, (const float*)h->ones.p, EDHMC_F32, st));
+  EDHMC_TRY(dev_alloc(ctx, h->offsets, (size_t)(G + 1) * 8, false));
+  if (hipMemcpyAsync(h->offsets.p, offsets, (size_t)(G + 1) * 8, hipMemcpyDeviceToDevice, st) !=
+      hipSuccess)
+    return set_err(ctx, EDHMC_EHIP, "copy offsets");
+  EDHMC_TRY(dev_alloc(ctx, h->gidx, (size_t)ctx->N_pad * 4, false));
+  hipLaunchKernelGGL(group_index_kernel, dim3(G), dim3(256), 0, st,
+                     (const int64_t*)h->offsets.p, G, ctx->N_pad, (int*)h->gidx.p);
+  EDHMC_TRY(check_launch(ctx, "group_index"));
+  EDHMC_TRY(dev_alloc(ctx, h->gidxp, (size_t)ctx->N_pad * 4, false));
+  EDHMC_TRY(rows_permute(ctx, h->gidx.p, ctx->N_pad, h->gidxp.p, st));
+  if (hipStreamSynchronize(st) != hipSuccess) return set_err(ctx, EDHMC_EHIP, "sync");
+  return EDHMC_OK;
+}
+
+}  // namespace edhmc
+
 using namespace edhmc;
 
 extern "C" {
@@ -449,34 +485,13 @@ int edhmc_bind_hier(edhmc_ctx* ctx, const float* X, const float* y, const int64_
     if (off[g + 1] < off[g]) return set_err(ctx, EDHMC_EINVAL, "offsets must be non-decreasing");
   if (ctx->hier) hier_destroy(ctx->hier);
   ctx->hier = nullptr;
-  HierModel* h = new (std::nothrow) HierModel();
-  if (!h) return set_err(ctx, EDHMC_ENOMEM, "host allocation");
-  ctx->hier = h;
-  h->G = G;
-  h->D = D;
-  h->N = N;
-  h->dim = G + 2 + D;
-  h->dim_pad = (int)round_up(h->dim, 4);
-  // w ~ N(0, I): the GLM prior for the shared coefficients
-  EDHMC_TRY(dev_alloc(ctx, h->ones, (size_t)D * 4, false));
-  EDHMC_TRY(dev_alloc(ctx, h->zeros, (size_t)D * 4));
-  std::vector<float> one(D, 1.0f);
-  if (hipMemcpyAsync(h->ones.p, one.data(), (size_t)D * 4, hipMemcpyHostToDevice, st) != hipSuccess)
-    return set_err(ctx, EDHMC_EHIP, "copy");
-  EDHMC_TRY(edhmc_bind_glm(ctx, X, EDHMC_F32, y, N, D, EDHMC_LIK_BERNOULLI, 1.0f,
-                           (const float*)h->zeros.p, (const float*)h->ones.p, EDHMC_F32, stream));
-  EDHMC_TRY(dev_alloc(ctx, h->offsets, (size_t)(G + 1) * 8, false));
-  if (hipMemcpyAsync(h->offsets.p, offsets, (size_t)(G + 1) * 8, hipMemcpyDeviceToDevice, st) !=
-      hipSuccess)
-    return set_err(ctx, EDHMC_EHIP, "copy offsets");
-  EDHMC_TRY(dev_alloc(ctx, h->gidx, (size_t)ctx->N_pad * 4, false));
-  hipLaunchKernelGGL(group_index_kernel, dim3(G), dim3(256), 0, st,
-                     (const int64_t*)h->offsets.p, G, ctx->N_pad, (int*)h->gidx.p);
-  EDHMC_TRY(check_launch(ctx, "group_index"));
-  EDHMC_TRY(dev_alloc(ctx, h->gidxp, (size_t)ctx->N_pad * 4, false));
-  EDHMC_TRY(rows_permute(ctx, h->gidx.p, ctx->N_pad, h->gidxp.p, st));
-  if (hipStreamSynchronize(st) != hipSuccess) return set_err(ctx, EDHMC_EHIP, "sync");
-  return EDHMC_OK;
+  const int rc = hier_bind_data(ctx, X, y, offsets, G, N, D, st);
+  if (rc != EDHMC_OK) {   // no model, rather than a part of one
+    if (ctx->hier) hier_destroy(ctx->hier);
+    ctx->hier = nullptr;
+    ctx->bound = false;
+  }
+  return rc;
 }
 
 int edhmc_hier_set_scale_prior(edhmc_ctx* ctx, int32_t kind, double p1, double p2,

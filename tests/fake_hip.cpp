@@ -22,6 +22,7 @@ std::map<const void*, std::string>& names() {   // used while libraries load
 std::set<void*> capturing;
 std::string lines, fail_kernel;
 size_t limit = SIZE_MAX, in_use = 0;
+int fail_malloc = 0;
 int error = 0;
 Config config;
 constexpr size_t kCopy = 1 << 20;   // larger memory is neither filled nor copied
@@ -38,6 +39,8 @@ const char* fake_log() { return lines.c_str(); }
 void fake_clear() { lines.clear(); }
 void fake_limit(size_t bytes) { limit = bytes; }
 size_t fake_in_use() { return in_use; }
+void fake_fail_malloc(int nth) { fail_malloc = nth; }   // 1: the next one; 0: none
+int fake_to_fail() { return fail_malloc; }
 void fake_capture(void* stream, int on) {
   if (on) capturing.insert(stream);
   else capturing.erase(stream);
@@ -47,7 +50,7 @@ void fake_fail_kernel(const char* part_of_name) { fail_kernel = part_of_name; }
 // -- the runtime's ------------------------------------------------------------
 int hipMalloc(void** p, size_t n) {
   *p = nullptr;
-  if (n > limit - in_use || in_use > limit) {
+  if (n > limit - in_use || in_use > limit || (fail_malloc > 0 && --fail_malloc == 0)) {
     log("malloc_failed " + std::to_string(n));
     return error = 2;
   }
