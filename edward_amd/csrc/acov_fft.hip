@@ -16,6 +16,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "common.h"
 #include "ctx.h"
@@ -134,17 +135,18 @@ struct Fft {
   }
 };
 
-// Columns k0 .. k0 + kc - 1 of s as rows of st [kc][Tp], and their means.
+// The series of kc / db chains and db coordinates, chains D columns of s
+// [T][K] apart, as rows of st [kc][Tp], and their means [chain][ldm].
 __global__ void __launch_bounds__(256)
-acov_rows_kernel(const float* __restrict__ s, int64_t T, int64_t K, int64_t k0, int64_t kc,
-                 int64_t Tp, float* __restrict__ st, double* __restrict__ mean) {
+acov_rows_kernel(const float* __restrict__ s, int64_t T, int64_t K, int D, int64_t kc, int db,
+                 int64_t Tp, float* __restrict__ st, double* __restrict__ mean, int64_t ldm) {
   __shared__ float tile[64][65];
   __shared__ double sum[4][64];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t c0 = (int64_t)blockIdx.x * 64;
-  const int64_t col = min(c0 + lane, kc - 1);
-  const float* p = s + k0 + col;
+  const int col = (int)min(c0 + lane, kc - 1), chain = col / db, d = col - chain * db;
+  const float* p = s + (int64_t)chain * D + d;
   float v[16];
   auto load = [&](int64_t t0) {
 #pragma unroll
@@ -175,7 +177,7 @@ acov_rows_kernel(const float* __restrict__ s, int64_t T, int64_t K, int64_t k0, 
   sum[wave][lane] = a;
   __syncthreads();
   if (wave == 0 && c0 + lane < kc)
-    mean[k0 + c0 + lane] = (((sum[0][lane] + sum[1][lane]) + sum[2][lane]) + sum[3][lane]) / (double)T;
+    mean[chain * ldm + d] = (((sum[0][lane] + sum[1][lane]) + sum[2][lane]) + sum[3][lane]) / (double)T;
 }
 
 // Power spectra of the chain pairs of coordinate d, one workgroup per d and
@@ -186,7 +188,7 @@ acov_rows_kernel(const float* __restrict__ s, int64_t T, int64_t K, int64_t k0, 
 template <int LOG>
 __global__ void __launch_bounds__(Fft<LOG>::kThreads)
 acov_power_kernel(const float* __restrict__ st, int64_t T, int64_t Tp, int D, int chains,
-                  const double* __restrict__ mean, int groups, bool first,
+                  const double* __restrict__ mean, int64_t ldm, int groups, bool first,
                   double* __restrict__ part) {
   using X = Fft<LOG>;
   __shared__ __align__(16) cplx lds[X::F * X::N];
@@ -214,8 +216,8 @@ acov_power_kernel(const float* __restrict__ st, int64_t T, int64_t Tp, int D, in
   fetch(g * X::F);
   for (int q = g * X::F; q < pairs; q += step) {
     const int c = 2 * (q + slot);
-    const double mx = c < chains ? mean[(int64_t)c * D + d] : 0.0;
-    const double my = c + 1 < chains ? mean[(int64_t)(c + 1) * D + d] : 0.0;
+    const double mx = c < chains ? mean[c * ldm + d] : 0.0;
+    const double my = c + 1 < chains ? mean[(c + 1) * ldm + d] : 0.0;
     cplx v[8];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -233,11 +235,11 @@ acov_power_kernel(const float* __restrict__ st, int64_t T, int64_t Tp, int D, in
   for (int i = 0; i < 8; ++i) out[X::out(j, i)] = acc[i];
 }
 
-// acov[l][d] = sum over the parts, made symmetric, transformed back, / (N T).
+// acov[l * ld + d] = sum over the parts, made symmetric, transformed back, / (N T).
 template <int LOG>
 __global__ void __launch_bounds__(Fft<LOG>::kThreads)
 acov_lags_kernel(const double* __restrict__ part, int parts, int D, int64_t T, int n_lags,
-                 double* __restrict__ acov) {
+                 double* __restrict__ acov, int64_t ld) {
   using X = Fft<LOG>;
   __shared__ __align__(16) cplx lds[X::F * X::N];
   const int slot = threadIdx.x / X::TH, j = threadIdx.x % X::TH;
@@ -264,7 +266,7 @@ acov_lags_kernel(const double* __restrict__ part, int parts, int D, int64_t T, i
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const int l = X::out(j, i);
-    if (ok && l < n_lags) acov[(int64_t)l * D + d] = v[i].re / X::N / (double)T;
+    if (ok && l < n_lags) acov[l * ld + d] = v[i].re / X::N / (double)T;
   }
 }
 
@@ -313,37 +315,53 @@ ess_kernel(const double* __restrict__ acov, const double* __restrict__ spread, i
 }
 
 constexpr int64_t kStoreBytes = 256 << 20;   // transposed chains held at a time
-constexpr int64_t kPartBytes = 64 << 20;
+constexpr int64_t kPartBytes = 64 << 20;     // partial spectra
 
+// Spectra of a coordinate, F side by side: 16 KB, 32 from 1025 draws on.
 template <int LOG>
-int launch(edhmc_ctx* ctx, const float* s, int64_t T, int C, int D, int n_lags, double* mean,
-           double* acov, hipStream_t st) {
+constexpr int64_t spectra_bytes = (int64_t)Fft<LOG>::F * Fft<LOG>::N * 8;
+
+// Coordinates s points at the first of; D: coordinates of the store.
+template <int LOG>
+int launch(edhmc_ctx* ctx, const float* s, int64_t T, int C, int D, int db, int n_lags,
+           double* mean, int64_t ldm, double* acov, int64_t ld, hipStream_t st) {
   using X = Fft<LOG>;
-  const int64_t K = (int64_t)C * D, Tp = (T + 15) / 16 * 16;
+  const int64_t Tp = (T + 15) / 16 * 16;
   // an even number of chains at a time
-  int64_t chunk = std::max<int64_t>(2, kStoreBytes / (Tp * 4 * D)) & ~1LL;
+  int64_t chunk = std::max<int64_t>(2, kStoreBytes / (Tp * 4 * db)) & ~1LL;
   chunk = std::min<int64_t>(chunk, C);
   const int64_t sets = ((chunk + 1) / 2 + X::F - 1) / X::F;   // of F pairs
-  int64_t groups = std::max<int64_t>(1, 4096 / D);            // two rounds of eight per unit
-  groups = std::min(groups, std::max<int64_t>(1, kPartBytes / ((int64_t)X::F * D * X::N * 8)));
+  int64_t groups = std::max<int64_t>(1, 4096 / db);           // two rounds of eight per unit
+  groups = std::min(groups, std::max<int64_t>(1, kPartBytes / (db * spectra_bytes<LOG>)));
   groups = std::min(groups, sets);
-  EDHMC_TRY(dev_reserve(ctx, ctx->acov_rows, (size_t)(chunk * D * Tp) * 4));
-  EDHMC_TRY(dev_reserve(ctx, ctx->acov_part, (size_t)(groups * X::F * D) * X::N * 8));
+  EDHMC_TRY(dev_reserve(ctx, ctx->acov_rows, (size_t)(chunk * db * Tp) * 4));
+  EDHMC_TRY(dev_reserve(ctx, ctx->acov_part, (size_t)(groups * db * spectra_bytes<LOG>)));
   float* rows = (float*)ctx->acov_rows.p;
   double* part = (double*)ctx->acov_part.p;
   for (int64_t c0 = 0; c0 < C; c0 += chunk) {
-    const int64_t cc = std::min<int64_t>(chunk, C - c0), kc = cc * D;
-    hipLaunchKernelGGL(acov_rows_kernel, dim3((unsigned)((kc + 63) / 64)), dim3(256), 0, st, s, T,
-                       K, c0 * D, kc, Tp, rows, mean);
+    const int64_t cc = std::min<int64_t>(chunk, C - c0), kc = cc * db;
+    hipLaunchKernelGGL(acov_rows_kernel, dim3((unsigned)((kc + 63) / 64)), dim3(256), 0, st,
+                       s + c0 * D, T, (int64_t)C * D, D, kc, db, Tp, rows, mean + c0 * ldm, ldm);
     EDHMC_TRY(check_launch(ctx, "acov_rows"));
-    hipLaunchKernelGGL((acov_power_kernel<LOG>), dim3((unsigned)(groups * D)), dim3(X::kThreads), 0,
-                       st, (const float*)rows, T, Tp, D, (int)cc, (const double*)mean + c0 * D,
-                       (int)groups, c0 == 0, part);
+    hipLaunchKernelGGL((acov_power_kernel<LOG>), dim3((unsigned)(groups * db)), dim3(X::kThreads),
+                       0, st, (const float*)rows, T, Tp, db, (int)cc,
+                       (const double*)mean + c0 * ldm, ldm, (int)groups, c0 == 0, part);
     EDHMC_TRY(check_launch(ctx, "acov_power"));
   }
-  hipLaunchKernelGGL((acov_lags_kernel<LOG>), dim3((D + X::F - 1) / X::F), dim3(X::kThreads), 0, st,
-                     (const double*)part, (int)(groups * X::F), D, T, n_lags, acov);
+  hipLaunchKernelGGL((acov_lags_kernel<LOG>), dim3((db + X::F - 1) / X::F), dim3(X::kThreads), 0,
+                     st, (const double*)part, (int)(groups * X::F), db, T, n_lags, acov, ld);
   return check_launch(ctx, "acov_lags");
+}
+
+template <typename F>
+auto with_log(int64_t T, F f) {
+  using std::integral_constant;
+  if (T <= 64) return f(integral_constant<int, 7>{});
+  if (T <= 128) return f(integral_constant<int, 8>{});
+  if (T <= 256) return f(integral_constant<int, 9>{});
+  if (T <= 512) return f(integral_constant<int, 10>{});
+  if (T <= 1024) return f(integral_constant<int, 11>{});
+  return f(integral_constant<int, 12>{});
 }
 
 }  // namespace
@@ -356,15 +374,22 @@ constexpr int64_t kFftMaxT = 2048;   // 4096 points of 16 bytes in LDS
 // 302; T = 1000, one chain, D = 10 174 / 35.
 bool autocov_fft_ok(int64_t T, int n_lags) { return T <= kFftMaxT && n_lags > 32; }
 
-// mean [C][D] is written too.
-int autocov_fft(edhmc_ctx* ctx, const float* s, int64_t T, int C, int D, int n_lags, double* mean,
-                double* acov, hipStream_t st) {
-  if (T <= 64) return launch<7>(ctx, s, T, C, D, n_lags, mean, acov, st);
-  if (T <= 128) return launch<8>(ctx, s, T, C, D, n_lags, mean, acov, st);
-  if (T <= 256) return launch<9>(ctx, s, T, C, D, n_lags, mean, acov, st);
-  if (T <= 512) return launch<10>(ctx, s, T, C, D, n_lags, mean, acov, st);
-  if (T <= 1024) return launch<11>(ctx, s, T, C, D, n_lags, mean, acov, st);
-  return launch<12>(ctx, s, T, C, D, n_lags, mean, acov, st);
+// Coordinates a call takes: as many as leave the transposed chains (two at
+// least) and the spectra (one group) within their bytes, in equal blocks.
+int autocov_fft_block(int64_t T, int D) {
+  const int64_t spec = with_log(T, [](auto lg) { return spectra_bytes<decltype(lg)::value>; });
+  const int64_t most = std::min(kPartBytes / spec, kStoreBytes / (2 * 4 * ((T + 15) / 16 * 16)));
+  const int64_t blocks = (D + most - 1) / most;
+  return (int)((D + blocks - 1) / blocks);
+}
+
+// Coordinates d0 .. d0 + db - 1, at most a block: their lags to acov [n_lags][ld]
+// and means to mean [C][ldm].
+int autocov_fft(edhmc_ctx* ctx, const float* s, int64_t T, int C, int D, int d0, int db, int n_lags,
+                double* mean, int64_t ldm, double* acov, int64_t ld, hipStream_t st) {
+  return with_log(T, [&](auto lg) {
+    return launch<decltype(lg)::value>(ctx, s + d0, T, C, D, db, n_lags, mean, ldm, acov, ld, st);
+  });
 }
 
 int ess_launch(edhmc_ctx* ctx, const double* acov, const double* mean, int64_t T, int C, int D,

@@ -15,8 +15,9 @@ using namespace edhmc;
 
 namespace edhmc {
 bool autocov_fft_ok(int64_t T, int n_lags);
-int autocov_fft(edhmc_ctx* ctx, const float* s, int64_t T, int C, int D, int n_lags, double* mean,
-                double* acov, hipStream_t st);
+int autocov_fft_block(int64_t T, int D);
+int autocov_fft(edhmc_ctx* ctx, const float* s, int64_t T, int C, int D, int d0, int db, int n_lags,
+                double* mean, int64_t ldm, double* acov, int64_t ld, hipStream_t st);
 int ess_launch(edhmc_ctx* ctx, const double* acov, const double* mean, int64_t T, int C, int D,
                bool between, double* ess, hipStream_t st);
 }  // namespace edhmc
@@ -136,6 +137,7 @@ int launch_moments(edhmc_ctx* ctx, const P* x, int64_t T, int64_t K, int64_t t0,
 // straight in the output, and with OWN_MEAN the chain means made here.
 // ---------------------------------------------------------------------------
 constexpr int kAcLags = 32, kAcStep = 8, kAcWaves = 4;
+constexpr int64_t kAcPartBytes = 128 << 20;     // partial sums
 constexpr int kAcWin = kAcLags / kAcStep + 1;   // window of kAcWin kAcStep values
 
 struct AcovArgs {
@@ -284,13 +286,22 @@ int autocov_lags(edhmc_ctx* ctx, const float* s, int64_t T, int C, int D, int la
     a.groups = (int)((a.blocks + per - 1) / per);
   };
   const int m = std::max(1, std::min(C, 64 / D));
+  const int64_t most = kAcPartBytes / ((int64_t)D * m * 8);   // lags of one group's partial sums
+  if (m > 1 && n_lags > most) {
+    for (int64_t l = 0; l < n_lags; l += most)
+      EDHMC_TRY(autocov_lags(ctx, s, T, C, D, (int)(lag0 + l), (int)std::min(most, n_lags - l), mean,
+                             acov + l * D, scratch, st));
+    return EDHMC_OK;
+  }
   // eight rounds of the 2048 waves that run together, so that the shorter
-  // sums of the long lags even out; at most 128 MB of partial sums
+  // sums of the long lags even out
   const int64_t strips = ((int64_t)D * m + 63) / 64;
   int64_t groups = std::max<int64_t>(1, 16384 / (strips * a.lag_wgs * kAcWaves));
-  groups = std::min<int64_t>(groups, std::max<int64_t>(1, (128 << 20) / ((int64_t)n_lags * D * m * 8)));
+  groups = std::min<int64_t>(groups, std::max<int64_t>(1, most / n_lags));
   split(m, groups);
-  if (scratch && dev_reserve(ctx, ctx->acov_part, (size_t)a.groups * n_lags * a.P * 8) == EDHMC_OK) {
+  if (a.m * a.groups == 1) {
+    a.part = acov;
+  } else if (scratch && dev_reserve(ctx, ctx->acov_part, (size_t)a.groups * n_lags * a.P * 8) == EDHMC_OK) {
     a.part = (double*)ctx->acov_part.p;
   } else {
     split(1, 1);
@@ -315,8 +326,12 @@ int autocov_from_zero(edhmc_ctx* ctx, const float* s, int64_t T, int C, int D, i
   if (!mean && scratch && dev_reserve(ctx, ctx->acov_mean, (size_t)C * D * 8) == EDHMC_OK)
     mean = (double*)ctx->acov_mean.p;
   if (mean && scratch && autocov_fft_ok(T, n_lags)) {
-    const int rc = autocov_fft(ctx, s, T, C, D, n_lags, mean, acov, st);
-    if (rc != EDHMC_ENOMEM) return rc;   // (before it has launched anything)
+    const int block = autocov_fft_block(T, D);
+    int rc = EDHMC_OK;
+    for (int d = 0; d < D && rc == EDHMC_OK; d += block)
+      rc = autocov_fft(ctx, s, T, C, D, d, std::min(block, D - d), n_lags, mean + d, D, acov + d, D,
+                       st);
+    if (rc != EDHMC_ENOMEM) return rc;
   }
   if (mean) EDHMC_TRY(launch_moments<float>(ctx, s, T, (int64_t)C * D, 0, mean, nullptr, st));
   return autocov_lags(ctx, s, T, C, D, 0, n_lags, mean, acov, scratch, st);
@@ -401,6 +416,19 @@ int edhmc_ess(edhmc_ctx* ctx, const float* s, int64_t T, int32_t C, int32_t D, i
   EDHMC_TRY(turn.begin());
   if (!turn.on) return set_err(ctx, EDHMC_EUNSUPPORTED, "edhmc_ess cannot be captured in a graph");
   auto go = [&]() -> int {
+    if (autocov_fft_ok(T, (int)T)) {   // the lags of a block of coordinates at a time
+      const int block = autocov_fft_block(T, D);
+      EDHMC_TRY(dev_reserve(ctx, ctx->acov_mean, (size_t)C * block * 8));
+      EDHMC_TRY(dev_reserve(ctx, ctx->acov, (size_t)T * block * 8));
+      double* mean = (double*)ctx->acov_mean.p;
+      double* acov = (double*)ctx->acov.p;
+      for (int d = 0; d < D; d += block) {
+        const int db = std::min(block, D - d);
+        EDHMC_TRY(autocov_fft(ctx, s, T, C, D, d, db, (int)T, mean, db, acov, db, st));
+        EDHMC_TRY(ess_launch(ctx, acov, mean, T, C, db, between != 0, ess_out + d, st));
+      }
+      return EDHMC_OK;
+    }
     EDHMC_TRY(dev_reserve(ctx, ctx->acov_mean, (size_t)C * D * 8));
     EDHMC_TRY(dev_reserve(ctx, ctx->acov, (size_t)T * D * 8));
     double* mean = (double*)ctx->acov_mean.p;

@@ -327,8 +327,10 @@ int edhmc_draw_uniforms(edhmc_ctx* ctx, int32_t C, uint64_t seed, uint64_t count
  *   acov_out   [max_lag+1, D] fp64  sum over chains of the biased (/T)
  *              within-chain autocovariance at each lag
  *   chain_mean [C, D] fp64 (may be NULL to skip)
- * This call and the two below share scratch that the context keeps: calls on
- * several streams take turns with it (each waits on the device for the one
+ * This call and the two below share scratch that the context keeps, at most
+ * 256 MB of transposed chains and 128 MB of partial sums or spectra, beside the
+ * chain means where the caller does not take them and, for edhmc_ess, the lags
+ * (32 MB up to 2048 draws, T D 8 bytes beyond): calls on several streams take turns with it (each waits on the device for the one
  * before).  In a stream capture the two autocovariance calls do without, one
  * group of chains after the other, as they do where the device has no memory
  * for it; edhmc_ess refuses a capturing stream (EDHMC_EUNSUPPORTED).        */
