@@ -98,11 +98,13 @@ constexpr int cmax(int a, int b) { return a > b ? a : b; }
 // chains are padded to a multiple of every M tile (and of the 128-row MLP
 // batch tile); data rows to a multiple of every row tile
 constexpr int kChainPad = cmax(cmax(Cfg1::BM, CfgG2::BM), cmax(CfgP2::BM, 128));
-constexpr int kRowPad = cmax(cmax(Cfg1::BN, CfgP2::BN), 128);
+constexpr int kRowPad = cmax(cmax(Cfg1::BN, CfgP2::BN), kFewRows);
 static_assert(kChainPad % Cfg1::BM == 0 && kChainPad % CfgG2::BM == 0 &&
               kChainPad % CfgP2::BM == 0 && kChainPad % 128 == 0, "chain padding");
 static_assert(Cfg1::kWN == 2 && Cfg1::kWavesN == 2 && Cfg1::BN == kLLTile, "order of the log-likelihood sums");
-static_assert(kRowPad % Cfg1::BN == 0 && kRowPad % CfgP2::BN == 0, "row padding");
+static_assert(kRowPad % Cfg1::BN == 0 && kRowPad % CfgP2::BN == 0 && kRowPad % kFewRows == 0,
+              "row padding");
+static_assert(kRowPad <= 2 * kLLTile, "rows_ll_kernel: at most one tile of padding");
 constexpr int kChainThreads = 256;
 
 // ---------------------------------------------------------------------------

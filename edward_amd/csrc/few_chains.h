@@ -50,6 +50,8 @@ struct FewArgs {
 
 // 16-row blocks per wave and tile: tiles of about 16 KB.
 constexpr int few_rb(int DP) { return DP <= 16 ? 4 : DP <= 32 ? 2 : 1; }
+// Whole tiles of X and y are read: N_pad is a multiple of the longest one.
+constexpr int kFewRows = 16 * few_rb(16) * kFewWaves;
 
 template <int DP, bool GRAD, bool LL>
 __global__ void __launch_bounds__(kFewThreads) __attribute__((amdgpu_waves_per_eu(1)))
@@ -64,6 +66,7 @@ few_chains_kernel(FewArgs a) {
   constexpr int C4 = DP / 4;                // float4 per row
   constexpr int PER_T = TR * C4 / NT;       // float4 per thread and tile
   static_assert(TR * C4 % NT == 0 && NG == 4 * G4 + 2 * G2 + G1, "tile");
+  static_assert(kFewRows % TR == 0, "tiles fill the padded rows");
   constexpr int XBUF = TR * S;
   constexpr int RED = GRAD ? kFewWaves * kFewTile * DP : 0;
   constexpr int SMF = 2 * XBUF > RED ? 2 * XBUF : RED;
@@ -91,7 +94,7 @@ few_chains_kernel(FewArgs a) {
   double lls = 0.0;
 
   // tile t: TR whole rows of X, one tile in registers ahead of the one in LDS
-  // (N_pad is a multiple of every TR: the last tile ends inside X and y)
+  // (N_pad is a multiple of kFewRows: the last tile ends inside X and y)
   f32x4_t pre[PER_T];
   float ypre = 0.0f;
   auto load = [&](int t) {
