@@ -25,6 +25,7 @@ namespace edhmc {
 
 int moments_f64(edhmc_ctx* ctx, const double* x, int64_t T, int64_t K, double* mean, double* var,
                 hipStream_t st);
+int sum_rows_f64(edhmc_ctx* ctx, double* p, int64_t rows, int64_t cols, hipStream_t st);
 
 namespace {
 
@@ -348,8 +349,16 @@ int launch(edhmc_ctx* ctx, const float* s, int64_t T, int C, int D, int db, int 
                        (const double*)mean + c0 * ldm, ldm, (int)groups, c0 == 0, part);
     EDHMC_TRY(check_launch(ctx, "acov_power"));
   }
+  int parts = (int)(groups * X::F);
+  // many chains of few coordinates: too long a chain of loads for the few
+  // workgroups of the next kernel (T = 100, 4096 chains, D = 10, effective
+  // sample sizes: 1470 -> 97 us; with 16 parts both are alike)
+  if (parts > 16) {
+    EDHMC_TRY(sum_rows_f64(ctx, part, parts, (int64_t)db * X::N, st));
+    parts = 1;
+  }
   hipLaunchKernelGGL((acov_lags_kernel<LOG>), dim3((db + X::F - 1) / X::F), dim3(X::kThreads), 0,
-                     st, (const double*)part, (int)(groups * X::F), db, T, n_lags, acov, ld);
+                     st, (const double*)part, parts, db, T, n_lags, acov, ld);
   return check_launch(ctx, "acov_lags");
 }
 
@@ -368,10 +377,12 @@ auto with_log(int64_t T, F f) {
 
 constexpr int64_t kFftMaxT = 2048;   // 4096 points of 16 bytes in LDS
 
-// From 33 lags on: the direct kernel (with its moments pass) takes two blocks of
-// 32 lags then.  us with 32 lags directly / all lags here: T = 1000, C = 1024,
-// D = 256 1459 / 1284; T = 2000, 1024, 128 1454 / 1683; T = 200, 1024, 256 570 /
-// 302; T = 1000, one chain, D = 10 174 / 35.
+// From 33 lags on, where the direct kernel takes a second block of 32.  us of a
+// call, 32 lags directly / 64 directly / all here: T = 1000, C = 1024, D = 256
+// 723 / 1165 / 1281; T = 2000, 1024, 128 718 / 1165 / 1678; T = 200, 1024, 256
+// 180 / 300 / 271; T = 100, 4096, 10 62 / 68 / 60; T = 1000, one chain, D = 10
+// 178 / 219 / 36.  (Up to 64 lags of long chains in a wide store the direct
+// kernel would still be ahead.)
 bool autocov_fft_ok(int64_t T, int n_lags) { return T <= kFftMaxT && n_lags > 32; }
 
 // Coordinates a call takes: as many as leave the transposed chains (two at

@@ -122,23 +122,22 @@ int launch_moments(edhmc_ctx* ctx, const P* x, int64_t T, int64_t K, int64_t t0,
 // a = x - chain mean, in FP64.
 //
 // A lane owns one column v of P = D m adjacent ones (m chains side by side,
-// so that narrow stores fill a wave) and 32 lags, whose sums stay in
-// registers over all the chains of its group.  Per step of 8 draws it loads
-// 8 new a_t and 8 new a_{t + lag} (the window of 40 rotates through five
-// register arrays) and issues 256 FP64 FMAs; the four waves of a workgroup
-// take adjacent lag blocks of the same columns, and the workgroups of one
-// column strip and chain group run on one XCD, so the store is read from its
-// L2.  Bound by the FP64 FMAs (n_lags (T - lag) C D of them) and the wait
-// for the loads.  T = 1000, C = 1024, D = 256, all 1000 lags in five windows:
-// 14.8 ms, against 105 ms for a thread per series with one atomic per series
-// and lag.  It takes windows that do not begin at lag 0, at most 32 lags, and
-// more than 2048 draws (acov_fft.hip the others), and whatever has to do
-// without scratch: then one group, chains one after the other, its sums
-// straight in the output, and with OWN_MEAN the chain means made here.
+// so that narrow stores fill a wave) and LAGS lags, whose sums stay in
+// registers over all the chains of its group.  With 32 lags, per step of 8
+// draws it loads 8 new a_t and 8 new a_{t + lag} (the window of 40 rotates
+// through five register arrays) and issues 256 FP64 FMAs; the waves of a
+// workgroup take adjacent lag blocks of the same columns, and the workgroups
+// of one column strip and chain group run on one XCD, so the store is read
+// from its L2.  Bound by the FP64 FMAs (n_lags (T - lag) C D of them) and the
+// wait for the loads.  T = 1000, C = 1024, D = 256, all 1000 lags in five
+// windows: 14.8 ms, against 105 ms for a thread per series with one atomic per
+// series and lag.  It takes windows that do not begin at lag 0, at most 32
+// lags, and more than 2048 draws (acov_fft.hip the others), and whatever has
+// to do without scratch: then one group, chains one after the other, its sums
+// straight in the output.  OWN_MEAN: it makes the chain means itself.
 // ---------------------------------------------------------------------------
-constexpr int kAcLags = 32, kAcStep = 8, kAcWaves = 4;
+constexpr int kAcStep = 8, kAcWaves = 4;
 constexpr int64_t kAcPartBytes = 128 << 20;     // partial sums
-constexpr int kAcWin = kAcLags / kAcStep + 1;   // window of kAcWin kAcStep values
 
 struct AcovArgs {
   const float* s;
@@ -147,13 +146,14 @@ struct AcovArgs {
   int lag0, n_lags;
   int blocks, groups;      // chain blocks of m chains, groups of them
   int strips, lag_wgs;     // 64-column strips of P, workgroups along the lags
-  const double* mean;      // [C][D] (OWN_MEAN: not read)
+  double* mean;            // [C][D] (OWN_MEAN: written, or null)
   double* part;            // [groups][n_lags][P]
 };
 
-template <bool OWN_MEAN>
-__global__ void __launch_bounds__(64 * kAcWaves) __attribute__((amdgpu_waves_per_eu(1, 2)))
+template <int LAGS, bool OWN_MEAN>
+__global__ void __launch_bounds__(64 * kAcWaves) __attribute__((amdgpu_waves_per_eu(LAGS > 8 ? 1 : 4, LAGS > 8 ? 2 : 8)))
 autocov_kernel(AcovArgs a) {
+  constexpr int WIN = LAGS / kAcStep + 1;   // window of WIN kAcStep values
   // units (strip, chain group) dealt to the XCDs, all lags of a unit on one
   const int units = a.strips * a.groups;
   const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
@@ -163,17 +163,17 @@ autocov_kernel(AcovArgs a) {
   const int lane = threadIdx.x & 63;
   // uniform over the wave: times and row addresses stay in scalar registers
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int lb = (local % a.lag_wgs) * kAcWaves + wave;   // lag block of this wave
-  if (lb * kAcLags >= a.n_lags) return;
-  const int64_t l0 = (int64_t)a.lag0 + (int64_t)lb * kAcLags;
+  const int lb = (local % a.lag_wgs) * (blockDim.x >> 6) + wave;   // lag block of this wave
+  if (lb * LAGS >= a.n_lags) return;
+  const int64_t l0 = (int64_t)a.lag0 + (int64_t)lb * LAGS;
   const int v = strip * 64 + lane;
   const int j = v / a.D, d = v - j * a.D;
   const int64_t stride = (int64_t)a.C * a.D;
   const int64_t T = a.T;
 
-  double acc[kAcLags];
+  double acc[LAGS];
 #pragma unroll
-  for (int l = 0; l < kAcLags; ++l) acc[l] = 0.0;
+  for (int l = 0; l < LAGS; ++l) acc[l] = 0.0;
   const int per = (a.blocks + a.groups - 1) / a.groups;
   const int k1 = min(a.blocks, (grp + 1) * per);
   for (int k = grp * per; k < k1; ++k) {
@@ -187,13 +187,14 @@ autocov_kernel(AcovArgs a) {
 #pragma unroll 16
       for (int64_t t = 0; t < T; ++t) mean += (double)x_at(t);
       mean /= (double)T;
+      if (lb == 0 && a.mean) a.mean[(int64_t)c * a.D + d] = mean;
     } else {
       mean = a.mean[(int64_t)c * a.D + d];
     }
-    double w[kAcWin][kAcStep];
+    double w[WIN][kAcStep];
     // a_t at times past the last draw read as 0
 #pragma unroll
-    for (int q = 0; q < kAcWin - 1; ++q)
+    for (int q = 0; q < WIN - 1; ++q)
 #pragma unroll
       for (int i = 0; i < kAcStep; ++i) {
         const int64_t t = l0 + q * kAcStep + i;
@@ -207,7 +208,7 @@ autocov_kernel(AcovArgs a) {
 #pragma unroll
       for (int i = 0; i < kAcStep; ++i) {
         ra[i] = x_at(t + i);
-        rw[i] = x_at(t + l0 + kAcLags + i);
+        rw[i] = x_at(t + l0 + LAGS + i);
       }
     };
     fetch(0);
@@ -215,35 +216,63 @@ autocov_kernel(AcovArgs a) {
     auto step = [&](int64_t t, auto rc) {
       constexpr int r = decltype(rc)::value;
       double x[kAcStep];
-      const int64_t tw = t + l0 + kAcLags;
+      const int64_t tw = t + l0 + LAGS;
 #pragma unroll
       for (int i = 0; i < kAcStep; ++i) {
         x[i] = (double)ra[i] - mean;
-        w[(r + kAcWin - 1) % kAcWin][i] = tw + i < T ? (double)rw[i] - mean : 0.0;
+        w[(r + WIN - 1) % WIN][i] = tw + i < T ? (double)rw[i] - mean : 0.0;
       }
       if (t + kAcStep < t_end) fetch(t + kAcStep);
 #pragma unroll
       for (int i = 0; i < kAcStep; ++i)
 #pragma unroll
-        for (int l = 0; l < kAcLags; ++l) {
+        for (int l = 0; l < LAGS; ++l) {
           const int q = i + l;
-          acc[l] = fma(x[i], w[(r + q / kAcStep) % kAcWin][q % kAcStep], acc[l]);
+          acc[l] = fma(x[i], w[(r + q / kAcStep) % WIN][q % kAcStep], acc[l]);
         }
     };
     using std::integral_constant;
-    for (int64_t t = 0; t < t_end; t += kAcWin * kAcStep) {
+    static_assert(WIN == 2 || WIN == 5, "steps of a turn of the window");
+    for (int64_t t = 0; t < t_end; t += WIN * kAcStep) {
       step(t, integral_constant<int, 0>{});
       if (t + kAcStep < t_end) step(t + kAcStep, integral_constant<int, 1>{});
-      if (t + 2 * kAcStep < t_end) step(t + 2 * kAcStep, integral_constant<int, 2>{});
-      if (t + 3 * kAcStep < t_end) step(t + 3 * kAcStep, integral_constant<int, 3>{});
-      if (t + 4 * kAcStep < t_end) step(t + 4 * kAcStep, integral_constant<int, 4>{});
+      if constexpr (WIN == 5) {
+        if (t + 2 * kAcStep < t_end) step(t + 2 * kAcStep, integral_constant<int, 2>{});
+        if (t + 3 * kAcStep < t_end) step(t + 3 * kAcStep, integral_constant<int, 3>{});
+        if (t + 4 * kAcStep < t_end) step(t + 4 * kAcStep, integral_constant<int, 4>{});
+      }
     }
   }
   if (v >= a.P) return;
 #pragma unroll
-  for (int l = 0; l < kAcLags; ++l)
-    if (lb * kAcLags + l < a.n_lags)
-      a.part[((int64_t)grp * a.n_lags + lb * kAcLags + l) * a.P + v] = acc[l];
+  for (int l = 0; l < LAGS; ++l)
+    if (lb * LAGS + l < a.n_lags)
+      a.part[((int64_t)grp * a.n_lags + lb * LAGS + l) * a.P + v] = acc[l];
+}
+
+// Column sums of p [rows][cols], into its first row: 64 columns per workgroup,
+// the rows dealt to sixteen waves, whose sums are added in order.  For the
+// partial sums of many chains over few draws, hundreds of groups of which
+// would otherwise be one long chain of loads per lag and coordinate: T = 32,
+// 4096 chains, D = 10, six lags 940 -> 22 us.
+__global__ void __launch_bounds__(1024)
+sum_rows_kernel(double* p, int64_t rows, int64_t cols) {
+  __shared__ double sm[16][64];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t c = (int64_t)blockIdx.x * 64 + lane;
+  double s = 0.0;
+  if (c < cols) {
+#pragma unroll 8
+    for (int64_t r = wave; r < rows; r += 16) s += p[r * cols + c];
+  }
+  sm[wave][lane] = s;
+  __syncthreads();
+  if (wave == 0 && c < cols) {
+#pragma unroll
+    for (int w = 1; w < 16; ++w) s += sm[w][lane];
+    p[c] = s;
+  }
 }
 
 // acov[l][d] = sum over the groups and the m side-by-side chains, / T (in place
@@ -257,15 +286,38 @@ autocov_sum_kernel(const double* part, int groups, int n_lags, int m, int D, int
   const int d = (int)(i - l * D);
   const int64_t P = (int64_t)D * m;
   double s = 0.0;
-  for (int g = 0; g < groups; ++g)
-    for (int j = 0; j < m; ++j) s += part[((int64_t)g * n_lags + l) * P + (int64_t)j * D + d];
+  const int n = groups * m;   // in order, sixteen loads in flight, then four
+  int q = 0;
+  auto add = [&](auto count) {
+    constexpr int K = decltype(count)::value;
+    double v[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int g = (q + k) / m, j = q + k - g * m;
+      v[k] = part[((int64_t)g * n_lags + l) * P + (int64_t)j * D + d];
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) s += v[k];
+    q += K;
+  };
+  while (q + 16 <= n) add(std::integral_constant<int, 16>{});
+  while (q + 4 <= n) add(std::integral_constant<int, 4>{});
+  while (q < n) add(std::integral_constant<int, 1>{});
   acov[i] = s / (double)T;
+}
+
+int sum_rows(edhmc_ctx* ctx, double* p, int64_t rows, int64_t cols, hipStream_t st) {
+  const int64_t wgs = (cols + 63) / 64;
+  if (wgs > 2147483647LL) return set_err(ctx, EDHMC_EUNSUPPORTED, "too many columns");
+  hipLaunchKernelGGL(sum_rows_kernel, dim3((unsigned)wgs), dim3(1024), 0, st, p, rows, cols);
+  return check_launch(ctx, "sum_rows");
 }
 
 // scratch: whether the context's may be used (and grow); without it, and where
 // the device has no memory for it, the call does without.
+// own: the means are made on the way, and written to `mean` unless that is null.
 int autocov_lags(edhmc_ctx* ctx, const float* s, int64_t T, int C, int D, int lag0, int n_lags,
-                 const double* mean, double* acov, bool scratch, hipStream_t st) {
+                 double* mean, bool own, double* acov, bool scratch, hipStream_t st) {
   AcovArgs a;
   a.s = s;
   a.T = T;
@@ -274,8 +326,12 @@ int autocov_lags(edhmc_ctx* ctx, const float* s, int64_t T, int C, int D, int la
   a.lag0 = lag0;
   a.n_lags = n_lags;
   a.mean = mean;
-  const int lag_blocks = (n_lags + kAcLags - 1) / kAcLags;
-  a.lag_wgs = (lag_blocks + kAcWaves - 1) / kAcWaves;
+  // lags per wave: 8 where there are no more, a quarter of the products and
+  // registers of 32 (T = 16, 4096 chains, D = 600, six lags, with the means on
+  // the way and no idle waves: 362 -> 92 us)
+  const int lags = n_lags <= 8 ? 8 : 32;
+  const int lag_blocks = (n_lags + lags - 1) / lags, waves = std::min(kAcWaves, lag_blocks);
+  a.lag_wgs = (lag_blocks + waves - 1) / waves;
   auto split = [&](int m, int64_t most) {   // m chains side by side, at most that many groups
     a.m = m;
     a.P = D * m;
@@ -290,13 +346,13 @@ int autocov_lags(edhmc_ctx* ctx, const float* s, int64_t T, int C, int D, int la
   if (m > 1 && n_lags > most) {
     for (int64_t l = 0; l < n_lags; l += most)
       EDHMC_TRY(autocov_lags(ctx, s, T, C, D, (int)(lag0 + l), (int)std::min(most, n_lags - l), mean,
-                             acov + l * D, scratch, st));
+                             own, acov + l * D, scratch, st));
     return EDHMC_OK;
   }
   // eight rounds of the 2048 waves that run together, so that the shorter
   // sums of the long lags even out
   const int64_t strips = ((int64_t)D * m + 63) / 64;
-  int64_t groups = std::max<int64_t>(1, 16384 / (strips * a.lag_wgs * kAcWaves));
+  int64_t groups = std::max<int64_t>(1, 16384 / (strips * a.lag_wgs * waves));
   groups = std::min<int64_t>(groups, std::max<int64_t>(1, most / n_lags));
   split(m, groups);
   if (a.m * a.groups == 1) {
@@ -310,19 +366,33 @@ int autocov_lags(edhmc_ctx* ctx, const float* s, int64_t T, int C, int D, int la
   const int64_t units = (int64_t)a.strips * a.groups;
   const int64_t grid = (units + 7) / 8 * 8 * a.lag_wgs;
   if (grid > 2147483647LL) return set_err(ctx, EDHMC_EUNSUPPORTED, "autocov: store too wide");
-  const dim3 wgs((unsigned)grid), block(64 * kAcWaves);
-  if (mean) hipLaunchKernelGGL(autocov_kernel<false>, wgs, block, 0, st, a);
-  else hipLaunchKernelGGL(autocov_kernel<true>, wgs, block, 0, st, a);
+  const dim3 wgs((unsigned)grid), block(64 * waves);
+  if (lags == 8 && own) hipLaunchKernelGGL((autocov_kernel<8, true>), wgs, block, 0, st, a);
+  else if (lags == 8) hipLaunchKernelGGL((autocov_kernel<8, false>), wgs, block, 0, st, a);
+  else if (own) hipLaunchKernelGGL((autocov_kernel<32, true>), wgs, block, 0, st, a);
+  else hipLaunchKernelGGL((autocov_kernel<32, false>), wgs, block, 0, st, a);
   EDHMC_TRY(check_launch(ctx, "autocov"));
+  // (up to 128 terms autocov_sum_kernel adds them as fast as two launches)
+  if (a.groups > 1 && a.groups * a.m > 128) {
+    EDHMC_TRY(sum_rows(ctx, a.part, a.groups, (int64_t)n_lags * a.P, st));
+    a.groups = 1;
+  }
   const int64_t n = (int64_t)n_lags * D;
   hipLaunchKernelGGL(autocov_sum_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
                      (const double*)a.part, a.groups, n_lags, a.m, D, T, acov);
   return check_launch(ctx, "autocov_sum");
 }
 
+// Draws up to which the direct kernel makes the chain means itself, one pass
+// and one launch less (T = 16, 64 chains, D = 100, six lags: 21.4 -> 17.4 us);
+// of more draws the moments pass has more loads in flight.
+constexpr int64_t kOwnMeanT = 64;
+
 // Lags 0 .. n_lags - 1 and, if asked for, the chain means they take.
 int autocov_from_zero(edhmc_ctx* ctx, const float* s, int64_t T, int C, int D, int n_lags,
                       double* mean, double* acov, bool scratch, hipStream_t st) {
+  if (T <= kOwnMeanT && !(scratch && autocov_fft_ok(T, n_lags)))
+    return autocov_lags(ctx, s, T, C, D, 0, n_lags, mean, true, acov, scratch, st);
   if (!mean && scratch && dev_reserve(ctx, ctx->acov_mean, (size_t)C * D * 8) == EDHMC_OK)
     mean = (double*)ctx->acov_mean.p;
   if (mean && scratch && autocov_fft_ok(T, n_lags)) {
@@ -334,7 +404,7 @@ int autocov_from_zero(edhmc_ctx* ctx, const float* s, int64_t T, int C, int D, i
     if (rc != EDHMC_ENOMEM) return rc;
   }
   if (mean) EDHMC_TRY(launch_moments<float>(ctx, s, T, (int64_t)C * D, 0, mean, nullptr, st));
-  return autocov_lags(ctx, s, T, C, D, 0, n_lags, mean, acov, scratch, st);
+  return autocov_lags(ctx, s, T, C, D, 0, n_lags, mean, !mean, acov, scratch, st);
 }
 
 // A call's turn with the context's readout scratch: it begins when the call
@@ -371,6 +441,9 @@ namespace edhmc {
 int moments_f64(edhmc_ctx* ctx, const double* x, int64_t T, int64_t K, double* mean, double* var,
                 hipStream_t st) {
   return launch_moments<double>(ctx, x, T, K, 0, mean, var, st);
+}
+int sum_rows_f64(edhmc_ctx* ctx, double* p, int64_t rows, int64_t cols, hipStream_t st) {
+  return sum_rows(ctx, p, rows, cols, st);
 }
 }  // namespace edhmc
 
@@ -449,8 +522,8 @@ int edhmc_autocov_lags(edhmc_ctx* ctx, const float* s, int64_t T, int32_t C, int
     return set_err(ctx, EDHMC_EINVAL, "bad arguments");
   ScratchTurn turn{ctx, (hipStream_t)stream};
   EDHMC_TRY(turn.begin());
-  return turn.end(autocov_lags(ctx, s, T, C, D, lag0, n_lags, chain_mean, acov_out, turn.on,
-                               (hipStream_t)stream));
+  return turn.end(autocov_lags(ctx, s, T, C, D, lag0, n_lags, (double*)chain_mean, false, acov_out,
+                               turn.on, (hipStream_t)stream));
 }
 
 }  // extern "C"
