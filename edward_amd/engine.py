@@ -41,11 +41,25 @@ def require_gpu():
     raise RuntimeError('edward_amd needs a ROCm GPU (MI355X/gfx950); none is visible')
 
 
+_deferred = []   # contexts collected during a graph capture: (lib, handle, device)
+
+
+def _destroy(lib, h, device):
+  torch.cuda.synchronize(device)
+  lib.edhmc_destroy(h)
+
+
+def _destroy_deferred():
+  while _deferred and not torch.cuda.is_current_stream_capturing():
+    _destroy(*_deferred.pop())
+
+
 class Context(object):
   """An edhmc_ctx on one device."""
 
   def __init__(self, device=0):
     require_gpu()
+    _destroy_deferred()
     self.lib = L.load()
     self.device = torch.device('cuda', device)
     h = ctypes.c_void_p()
@@ -54,12 +68,17 @@ class Context(object):
 
   def close(self):
     if getattr(self, 'h', None):
-      torch.cuda.synchronize(self.device)
-      self.lib.edhmc_destroy(self.h)
+      _destroy(self.lib, self.h, self.device)
       self.h = None
+      _destroy_deferred()
 
   def __del__(self):
     try:
+      if getattr(self, 'h', None) and torch.cuda.is_current_stream_capturing():
+        # the collector may come at any time; waiting for the device would end
+        # the capture
+        _deferred.append((self.lib, self.h, self.device))
+        self.h = None
       self.close()
     except Exception:
       pass
