@@ -80,26 +80,30 @@ __device__ inline double block_sum_f64(double v, double* sm /* >= NT/64 */) {
   return t;
 }
 
-// Sum of p[q * stride], q < n, in order: sixteen loads in flight, then eight
-// (n is a multiple of 8 from 8 on in the gradient's partial sums), four, one.
-// A loop unrolled sixteen times took the eight of a small model one by one: 390
+// f(p[q * stride]) for q < n in order: sixteen loads in flight, then eight (n
+// is a multiple of 8 from 8 on in the gradient's partial sums), four, one.  A
+// loop unrolled sixteen times took the eight of a small model one by one: 390
 // chains on 2507 x 193, bf16, 498 us a transition of eleven steps, here 480.
-__device__ inline float strided_sum(const float* p, int64_t stride, int n) {
-  float s = 0.0f;
+template <typename F>
+__device__ inline void strided_each(const float* p, int64_t stride, int n, F f) {
   int q = 0;
-  auto add = [&](auto count) {
+  auto some = [&](auto count) {
     constexpr int K = decltype(count)::value;
     float v[K];
 #pragma unroll
     for (int i = 0; i < K; ++i) v[i] = p[(q + i) * stride];
 #pragma unroll
-    for (int i = 0; i < K; ++i) s += v[i];
+    for (int i = 0; i < K; ++i) f(v[i]);
     q += K;
   };
-  while (q + 16 <= n) add(std::integral_constant<int, 16>{});
-  if (q + 8 <= n) add(std::integral_constant<int, 8>{});
-  if (q + 4 <= n) add(std::integral_constant<int, 4>{});
-  while (q < n) add(std::integral_constant<int, 1>{});
+  while (q + 16 <= n) some(std::integral_constant<int, 16>{});
+  if (q + 8 <= n) some(std::integral_constant<int, 8>{});
+  if (q + 4 <= n) some(std::integral_constant<int, 4>{});
+  while (q < n) some(std::integral_constant<int, 1>{});
+}
+__device__ inline float strided_sum(const float* p, int64_t stride, int n) {
+  float s = 0.0f;
+  strided_each(p, stride, n, [&](float v) { s += v; });
   return s;
 }
 

@@ -380,7 +380,7 @@ colsum_reduce_kernel(const float* __restrict__ part, int m_tiles, int64_t ld, in
   const int64_t n = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (n >= N) return;
   double s = 0.0;
-  for (int t = 0; t < m_tiles; ++t) s += (double)part[(int64_t)t * ld + n];
+  strided_each(part + n, ld, m_tiles, [&](float v) { s += (double)v; });
   out[n] = (float)(s / (double)S);
 }
 

@@ -85,10 +85,18 @@ predict_kernel(PredictArgs a) {
   // chunk u of row r in slot u ^ swz(r): sixteen rows' chunks hit disjoint banks
   auto swz = [](int r) { return Q % 4 == 0 ? r & 15 : Q % 2 == 0 ? (r >> 1) & 7 : (r >> 2) & 3; };
 
-  // the draws' tiles of one row range run on one XCD and share its L2
-  const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
-  const int tile = local % a.tiles, split = xcd + 8 * (local / a.tiles);
-  if (split >= a.splits) return;
+  // the draws' tiles of one row range run on one XCD and share its L2; fewer
+  // ranges than XCDs are spread over all of them
+  int tile, split;
+  if (a.splits >= 8) {
+    const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
+    tile = local % a.tiles;
+    split = xcd + 8 * (local / a.tiles);
+    if (split >= a.splits) return;
+  } else {
+    tile = blockIdx.x % a.tiles;
+    split = blockIdx.x / a.tiles;
+  }
   LikParams lp = a.lp;
   lp.lik = BERN ? LIK_BERNOULLI : LIK_NORMAL;
   const int tid = threadIdx.x, lane = tid & 63;

@@ -22,8 +22,17 @@ PredictPlan predict_plan(const edhmc_ctx* ctx, int S) {
   p.wc = 10 * pad(4) <= 11 * pad(2) ? 4 : 2;
   p.tiles = (int)(pad(p.wc) / (p.wc * per));
   p.cols = p.tiles * p.wc;
-  // the workgroups that run together in one round, of at least 128 rows each
-  const int64_t want = std::max(1, (predict_q(ctx) <= 8 ? 1024 : 512) / p.tiles);
+  // as many ranges on every XCD as run together there in one round; where that
+  // leaves a fifth of it idle (thousands of draws), up to eight, so that the
+  // compute units' shares even out
+  const int slots = predict_q(ctx) <= 8 ? 128 : 64;
+  int each = std::max(1, slots / p.tiles);
+  if (5 * each * p.tiles < 4 * slots) {
+    auto share = [&](int e) { return (e * p.tiles + 31) / 32 / (double)e; };   // of a unit
+    for (int e = each + 1; e <= 8; ++e)
+      if (share(e) < share(each)) each = e;
+  }
+  const int64_t want = 8 * each;   // ranges, of at least 128 rows
   p.rows_per_split = std::max<int64_t>(128, round_up((ctx->N + want - 1) / want, 64));
   // a range is addressed with 31-bit byte offsets
   p.rows_per_split = std::min<int64_t>(p.rows_per_split, (0x7fffffffLL / (ctx->D_pad * 4) - 64) / 64 * 64);
@@ -33,7 +42,7 @@ PredictPlan predict_plan(const edhmc_ctx* ctx, int S) {
 
 template <int Q>
 static void launch_q(const PredictArgs& a, int wc, hipStream_t st) {
-  const dim3 grid(8 * ((a.splits + 7) / 8) * a.tiles), block(256);
+  const dim3 grid((a.splits >= 8 ? 8 * ((a.splits + 7) / 8) : a.splits) * a.tiles), block(256);
   const bool bern = a.lp.lik == LIK_BERNOULLI;
   auto go = [&](auto w) {
     constexpr int WC = decltype(w)::value;
