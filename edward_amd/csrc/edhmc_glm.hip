@@ -480,8 +480,10 @@ ll_final_kernel(const double* __restrict__ split, int C_pad, double* __restrict_
   ll[c] = s;
 }
 
+// perm (or null): the copy in grad_rows.h's row order (rows_permute's)
 __global__ void pad_copy_kernel(const float* __restrict__ src, int64_t n, float* __restrict__ dst,
-                                int64_t n_pad, float fill, int* nonfinite) {
+                                float* __restrict__ perm, int64_t n_pad, float fill,
+                                int* nonfinite) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n_pad) return;
   float v = fill;
@@ -490,6 +492,7 @@ __global__ void pad_copy_kernel(const float* __restrict__ src, int64_t n, float*
     if (!isfinite(v)) atomicAdd(nonfinite, 1);
   }
   dst[i] = v;
+  if (perm) perm[(i & ~15LL) + pi16_inv((int)(i & 15))] = v;
 }
 
 // ---------------------------------------------------------------------------
@@ -2376,15 +2379,14 @@ int edhmc_bind_glm(edhmc_ctx* ctx, const void* X, int32_t x_in_dtype, const floa
                        st, (const bf16_t*)ctx->Xr.p, pieces, ctx->D_pad, (bf16_t*)ctx->Xf.p);
     EDHMC_TRY(check_launch(ctx, "layout_frag"));
   }
-  auto padc = [&](const float* src, int64_t n, DevBuf& dst, int64_t npad, float fill) {
+  auto padc = [&](const float* src, int64_t n, DevBuf& dst, void* perm, int64_t npad, float fill) {
     hipLaunchKernelGGL(pad_copy_kernel, dim3((unsigned)((npad + 255) / 256)), dim3(256), 0, st,
-                       src, n, (float*)dst.p, npad, fill, bad);
+                       src, n, (float*)dst.p, (float*)perm, npad, fill, bad);
     return check_launch(ctx, "pad_copy");
   };
-  EDHMC_TRY(padc(y, N, ctx->y, ctx->N_pad, 0.0f));
-  if (ctx->yp.p) EDHMC_TRY(rows_permute(ctx, ctx->y.p, ctx->N_pad, ctx->yp.p, st));
-  EDHMC_TRY(padc(prior_loc, D, ctx->ploc, ctx->D_pad, 0.0f));
-  EDHMC_TRY(padc(prior_scale, D, ctx->pscale, ctx->D_pad, 1.0f));
+  EDHMC_TRY(padc(y, N, ctx->y, ctx->yp.p, ctx->N_pad, 0.0f));
+  EDHMC_TRY(padc(prior_loc, D, ctx->ploc, nullptr, ctx->D_pad, 0.0f));
+  EDHMC_TRY(padc(prior_scale, D, ctx->pscale, nullptr, ctx->D_pad, 1.0f));
   int nbad = 0;
   if (hipMemcpyAsync(&nbad, bad, 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
       hipStreamSynchronize(st) != hipSuccess)
