@@ -116,6 +116,7 @@ struct edhmc_ctx {
   edhmc::DevBuf Rt, Gpart, llpart, ll;
   int ksplit = 1;        // partial gradients in Gpart, g_ld chains x D_pad apart
   int64_t g_ld = 0;
+  bool rows_wide = false;   // form of the one-pass gradient (grad_rows.h)
   edhmc::FewPlan few;
   edhmc::DevBuf Xs;      // X with few.DP < D_pad columns (few-chain gradient)
   int n_tiles1 = 0;      // GEMM1 column tiles (= llpart leading dim)

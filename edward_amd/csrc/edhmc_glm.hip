@@ -1227,6 +1227,7 @@ static int rows_eval(edhmc_ctx* ctx, bool ll, hipStream_t st, const HierRows* hr
   a.rows_per_split = (stages + ctx->ksplit - 1) / ctx->ksplit * (kStageBytes / 4);
   a.C = ctx->C;
   a.splits = ctx->ksplit;
+  a.wide = ctx->rows_wide;
   a.lp = lik_params(ctx);
   a.Gpart = (float*)ctx->Gpart.p;
   a.g_ld = ctx->g_ld;
@@ -1243,7 +1244,7 @@ static int rows_eval(edhmc_ctx* ctx, bool ll, hipStream_t st, const HierRows* hr
     a.G = hr->G;
     a.Rt = (float*)ctx->Rt.p;
     a.ldr = ctx->C_pad;
-    *summed = rows_wide(a.C, a.splits) ? a.rows_per_split : 0;
+    *summed = a.wide ? a.rows_per_split : 0;
   }
   {
     ProfScope ps(ctx, PK_GEMM_GRAD, st);
@@ -2029,6 +2030,7 @@ static int alloc_chains(edhmc_ctx* ctx, int C, hipStream_t st) {
   EDHMC_TRY(dev_alloc(ctx, ctx->ratio, (size_t)C * 8));
   ctx->n_tiles1 = (int)(ctx->N_pad / std::min(Cfg1::BN, CfgP2::BN));   // llpart rows
   ctx->few = few_plan(ctx, C);
+  size_t eta_bytes = 0;
   if (ctx->few.on) {
     // no residuals: the row ranges' partial gradients of the C chains
     ctx->Rt.release();
@@ -2050,11 +2052,12 @@ static int alloc_chains(edhmc_ctx* ctx, int C, hipStream_t st) {
     if (ks >= 8) ks = ks / 8 * 8;
     ctx->ksplit = ks;
     ctx->g_ld = C_pad;
+    ctx->rows_wide = rows_wide(C, ks);
+    if (rows_ok(ctx)) eta_bytes = (size_t)rows_eta(C, ks, ctx->N_pad, ctx->rows_wide) * 4;
+    if (ctx->eta.bytes != eta_bytes) ctx->eta.release();
     // residuals: none after a one-pass gradient but the hierarchical model's;
     // rows up to a whole W-stationary tile, whose residual epilogue stores the
     // last tile's rows past N_pad (zeros) without a bounds test
-    if (rows_ok(ctx)) EDHMC_TRY(dev_alloc(ctx, ctx->eta, (size_t)rows_eta(C, ks, ctx->N_pad) * 4, false));
-    else ctx->eta.release();
     if (rows_ok(ctx) && !ctx->hier) ctx->Rt.release();
     else EDHMC_TRY(dev_alloc(ctx, ctx->Rt, (size_t)C_pad * round_up(ctx->N_pad, kWsTile) * eb, false));
   }
@@ -2062,6 +2065,16 @@ static int alloc_chains(edhmc_ctx* ctx, int C, hipStream_t st) {
   EDHMC_TRY(dev_alloc(ctx, ctx->llpart, (size_t)C_pad * ctx->n_tiles1 * 8, false));
   EDHMC_TRY(dev_alloc(ctx, ctx->ll, (size_t)C_pad * 8));
   EDHMC_TRY(dev_alloc(ctx, ctx->ll_split, (size_t)kLLSplit * C_pad * 8, false));
+  if (eta_bytes) {
+    int rc = dev_alloc(ctx, ctx->eta, eta_bytes, false);
+    if (rc == EDHMC_ENOMEM && !ctx->rows_wide) {
+      // the chain-split form keeps eta of far fewer rows: for where this one's
+      // does not fit beside the hierarchical model's residuals
+      ctx->rows_wide = true;
+      rc = dev_alloc(ctx, ctx->eta, (size_t)rows_eta(C, ctx->ksplit, ctx->N_pad, true) * 4, false);
+    }
+    return rc;
+  }
   return EDHMC_OK;
 }
 

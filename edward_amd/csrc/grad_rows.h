@@ -54,6 +54,7 @@ struct RowsArgs {
   int64_t N, N_pad;
   int64_t rows_per_split;  // multiple of 16
   int C, tiles, splits;
+  bool wide;               // grad_wide_kernel
   LikParams lp;
   float* Gpart;            // [splits][g_ld][DP]
   int64_t g_ld;
@@ -752,19 +753,19 @@ grad_wide_kernel(RowsArgs a) {
 // may come last.
 template <bool BERN>
 __global__ void __launch_bounds__(256)
-rows_ll_kernel(RowsArgs a, bool wide) {
+rows_ll_kernel(RowsArgs a) {
   const int l = threadIdx.x & 31, c = blockIdx.x * 8 + (threadIdx.x >> 5);
   if (c >= a.C) return;
   LikParams lp = a.lp;
   lp.lik = BERN ? LIK_BERNOULLI : LIK_NORMAL;
-  const int64_t tiles = a.N_pad / kLLTile, slots = wide ? a.splits + 1 : tiles;
+  const int64_t tiles = a.N_pad / kLLTile, slots = a.wide ? a.splits + 1 : tiles;
   for (int64_t slot = blockIdx.y; slot < slots; slot += gridDim.y) {
     int64_t tile = slot;
-    if (wide && slot < a.splits) {
+    if (a.wide && slot < a.splits) {
       const int64_t e = (slot + 1) * a.rows_per_split;   // in two ranges, of which this is the first
       tile = e / kLLTile;
       if (e % kLLTile == 0 || tile >= tiles || tile * kLLTile / a.rows_per_split != slot) continue;
-    } else if (wide) {
+    } else if (a.wide) {
       tile = tiles - 1;
       if (tile * kLLTile < a.N) continue;
     }
@@ -794,11 +795,12 @@ rows_ll_kernel(RowsArgs a, bool wide) {
 
 // Whether the bound data take this kernel (and bind makes Xp and yp).
 bool rows_ok(const edhmc_ctx* ctx);
-// Whether a call of C chains over this many row ranges takes grad_wide_kernel.
+// Whether a call of C chains over this many row ranges is faster with
+// grad_wide_kernel (the bits are the same).
 bool rows_wide(int C, int splits);
 // Floats that RowsArgs.eta holds.
-int64_t rows_eta(int C, int splits, int64_t N_pad);
-// Fills in the chain tiles (C, splits set) and launches.
+int64_t rows_eta(int C, int splits, int64_t N_pad, bool wide);
+// Fills in the chain tiles (C, splits, wide set) and launches.
 int rows_launch(edhmc_ctx* ctx, RowsArgs a, bool ll, hipStream_t st);
 // out[16 b + p] = in[16 b + pi(p)] for n values (a multiple of 16), 4 bytes each.
 int rows_permute(edhmc_ctx* ctx, const void* in, int64_t n, void* out, hipStream_t st);

@@ -57,7 +57,7 @@ static void launch_wide(RowsArgs a, bool ll, hipStream_t st) {
 
 template <int DP>
 static void launch_dp(const RowsArgs& a, bool ll, hipStream_t st) {
-  if (rows_wide(a.C, a.splits)) return launch_wide<DP>(a, ll, st);
+  if (a.wide) return launch_wide<DP>(a, ll, st);
   // 16 chains per workgroup while that leaves at most one (64 columns: two) per
   // compute unit.  us per step against 32 chains, N = 100,000, 64 ranges: D =
   // 60, 64 / 128 / 256 chains 32 / 45 / 80 and 47 / 48 / 74; D = 120, 64 / 128
@@ -69,8 +69,8 @@ static void launch_dp(const RowsArgs& a, bool ll, hipStream_t st) {
   launch_cw<DP, 2>(a, ll, st);
 }
 
-int64_t rows_eta(int C, int splits, int64_t N_pad) {
-  return rows_wide(C, splits) ? (int64_t)splits * C * kLLTile : N_pad * C;
+int64_t rows_eta(int C, int splits, int64_t N_pad, bool wide) {
+  return wide ? (int64_t)splits * C * kLLTile : N_pad * C;
 }
 
 int rows_launch(edhmc_ctx* ctx, RowsArgs a, bool ll, hipStream_t st) {
@@ -85,11 +85,10 @@ int rows_launch(edhmc_ctx* ctx, RowsArgs a, bool ll, hipStream_t st) {
   }
   EDHMC_TRY(check_launch(ctx, "grad_rows"));
   if (!ll) return EDHMC_OK;
-  const bool wide = rows_wide(a.C, a.splits);
-  const int64_t slots = wide ? a.splits + 1 : a.N_pad / kLLTile;
+  const int64_t slots = a.wide ? a.splits + 1 : a.N_pad / kLLTile;
   const dim3 grid((a.C + 7) / 8, (unsigned)std::min<int64_t>(slots, 4096));
-  if (a.lp.lik == LIK_BERNOULLI) hipLaunchKernelGGL((rows_ll_kernel<true>), grid, dim3(256), 0, st, a, wide);
-  else hipLaunchKernelGGL((rows_ll_kernel<false>), grid, dim3(256), 0, st, a, wide);
+  if (a.lp.lik == LIK_BERNOULLI) hipLaunchKernelGGL((rows_ll_kernel<true>), grid, dim3(256), 0, st, a);
+  else hipLaunchKernelGGL((rows_ll_kernel<false>), grid, dim3(256), 0, st, a);
   return check_launch(ctx, "rows_ll");
 }
 

@@ -45,6 +45,11 @@ while True:
     break
   failed = log()
   at = [l[0] for l in failed].index('malloc_failed')
+  if rc == 0:      # eta's: the form that needs less of it
+    assert any('grad_wide' in k for k in kernels(failed)), (n, failed)
+    lib.edhmc_destroy(h)
+    n += 1
+    continue
   assert rc == L.ENOMEM and not kernels(failed[at:]), (n, rc, failed)
   assert lib.edhmc_run(h, 0.1, 2, X, 3, 0, 3, 1, 0, None, None) == L.ESTATE
   assert lib.edhmc_moments_enable(h, 1) == L.ESTATE
@@ -117,6 +122,10 @@ while True:
     break
   failed = log()
   at = [l[0] for l in failed].index('malloc_failed')
+  if rc == 0:
+    assert any('grad_wide' in k for k in kernels(failed)), (n, failed)
+    n += 1
+    continue
   assert rc == L.ENOMEM and not kernels(failed[at:]), (n, rc, failed)
   assert lib.edhmc_hier_transition(h, 0.1, 2, None, None, 1, 0, None, None, None, None) == L.ESTATE
   log()
