@@ -1980,7 +1980,7 @@ static int launch_predict(edhmc_ctx* ctx, int S, bool want_mean, float* rep, uin
   g.stages_per_split = g.k_stages;
   g.swz = 1;
   if (!gemm_offsets_fit<Cfg, PLANES>(g)) return set_err(ctx, EDHMC_EUNSUPPORTED, "tile too large");
-  if (want_mean) EDHMC_TRY(dev_alloc(ctx, ctx->pred_col, (size_t)g.m_tiles * ctx->N_pad * 4, false));
+  if (want_mean) EDHMC_TRY(dev_reserve(ctx, ctx->pred_col, (size_t)g.m_tiles * ctx->N_pad * 4));
   EpiPredict<T> e;
   e.y = (const float*)ctx->y.p;
   e.N = ctx->N;
@@ -2505,7 +2505,7 @@ int edhmc_predict(edhmc_ctx* ctx, const float* W, int32_t S, float* mean_out, do
   if (predict_ok(ctx) && !rep_out) {   // replicates: the general kernel stores the mean responses
     const PredictPlan p = predict_plan(ctx, S);
     cols = p.cols;
-    if (mean_out) EDHMC_TRY(dev_alloc(ctx, ctx->pred_col, (size_t)cols * ctx->N_pad * 4, false));
+    if (mean_out) EDHMC_TRY(dev_reserve(ctx, ctx->pred_col, (size_t)cols * ctx->N_pad * 4));
     PredictArgs pa = {};
     pa.Xp = (const float*)ctx->Xp.p;
     pa.y = (const float*)ctx->y.p;

@@ -79,9 +79,9 @@ int hipMemsetAsync(void* p, int v, size_t n, void* st) {
   log("memset " + str(st));
   return hipMemset(p, v, n);
 }
-int hipMemcpyAsync(void* d, const void* s, size_t n, int, void* st) {
+int hipMemcpyAsync(void* d, const void* s, size_t n, int kind, void* st) {
   log("memcpy " + str(st));
-  if (n <= kCopy) memcpy(d, s, n);
+  if (kind != 3 && n <= kCopy) memcpy(d, s, n);   // not from device to device
   return 0;
 }
 int hipStreamSynchronize(void* st) {
