@@ -83,7 +83,7 @@ __device__ inline double block_sum_f64(double v, double* sm /* >= NT/64 */) {
 // f(p[q * stride]) for q < n in order: sixteen loads in flight, then eight (n
 // is a multiple of 8 from 8 on in the gradient's partial sums), four, one.  A
 // loop unrolled sixteen times took the eight of a small model one by one: 390
-// chains on 2507 x 193, bf16, 498 us a transition of eleven steps, here 480.
+// chains on 2507 x 193, bf16, 497 us a transition of eleven steps, here 483.
 template <typename F>
 __device__ inline void strided_each(const float* p, int64_t stride, int n, F f) {
   int q = 0;

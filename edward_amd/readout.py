@@ -1,7 +1,7 @@
 """Readout of Empirical sample stores (``edward/models/empirical.py:87-96``).
 
-Device stores are reduced by ``edhmc_sample_moments`` (two-pass FP64 on the
-GPU); a store the user keeps in host memory is reduced on the host in FP64,
+Device stores are reduced by ``edhmc_sample_moments`` (FP64 on the GPU, the
+store read once); a store the user keeps in host memory is reduced on the host in FP64,
 since it never reaches the device."""
 
 import numpy as np

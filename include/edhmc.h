@@ -268,7 +268,7 @@ int64_t edhmc_record_count(edhmc_ctx* ctx);
 
 /* Empirical.mean / Empirical.variance (edward/models/empirical.py:87-96) of a
  * sample store params [T, K] (K = product of the event shape) over rows
- * t0 .. T-1: two-pass FP64, divisor T - t0 (population variance, as the
+ * t0 .. T-1: FP64, read once, divisor T - t0 (population variance, as the
  * reference's stddev).  params_dtype EDHMC_F32 or 2 (= fp64);
  * mean_out, var_out [K] fp64. */
 int edhmc_sample_moments(edhmc_ctx* ctx, const void* params, int32_t params_dtype, int64_t T,
